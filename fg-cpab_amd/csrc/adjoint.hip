@@ -1,7 +1,7 @@
 // Fused backward: midpoint-trajectory replay + discrete adjoint + cell moments
 // (cpab_ops_1d.cu:331-422, cpab_ops_2d.cu:384-513, cpab_ops_3d.cu:405-532).
 //
-// Per trajectory (one lane), two variants:
+// Per trajectory (one lane), three variants:
 //   register  (T == kRegSteps) phase 1 runs the T explicit-midpoint steps
 //             fully unrolled and keeps every cell in VGPRs (two per
 //             register); phase 2 walks them backwards, recovering each
@@ -9,13 +9,18 @@
 //             (with adaptive substeps, whose steps are not fixed affine maps,
 //             the positions are kept in VGPRs too).  One midpoint pass per
 //             trajectory.
-//   segmented (any T <= 100) phase 1 keeps a checkpoint every kSeg steps in a
-//             VGPR shift register; phase 2 replays each segment from its
+//   trail     (any T, no adaptive substeps, up to 65535 cells) the same with
+//             the loops over the steps rolled in groups of kSeg: the groups'
+//             cells and start positions are written to and read from VGPRs
+//             at a wave-uniform index.
+//   segmented (any T <= 100; adaptive substeps, more cells, rows beyond the
+//             recovery bound) phase 1 keeps a checkpoint every kSeg steps in
+//             a VGPR shift register; phase 2 replays each segment from its
 //             checkpoint into registers and walks it backwards (the
 //             reference's scheme, cpab_ops_2d.cu:236-263).
-// Both visit the reference's cells; the positions fed to the sums may differ
-// from the replayed ones by a few ulps in the register variant.
-// In both, phase 2 propagates lambda and accumulates the 2x3 (1x2, 3x4) sum
+// All visit the reference's cells; the positions fed to the sums may differ
+// from the replayed ones by a few ulps in the register and trail variants.
+// In all, phase 2 propagates lambda and accumulates the 2x3 (1x2, 3x4) sum
 // S = sum lam (x) [p; 1] of the current cell, flushing it whenever the cell
 // changes, as the reference groups its moment flushes.  The reverse step is the
 // factored form of cpab_ops_2d.cu:334-382 (cpab_device.hpp, adjoint_s*): lam is
@@ -57,8 +62,7 @@
 namespace cpab {
 namespace {
 
-// TS == 0: segmented variant; TS > 0: register variant.  Both accumulate in
-// full LDS bins or the LDS cell cache.
+// BODY: the variant.  All accumulate in full LDS bins or the LDS cell cache.
 // One workgroup = one theta x one contiguous point range (wg_slot).  A chain
 // of K stages (Cpab.transform_grid_chain) runs its stages last to first
 // inside the kernel: stage k reads its input points from
@@ -69,16 +73,17 @@ namespace {
 // on entry), or, from a dense full-bin workgroup, to its partial table with
 // its dense-part bit set; the reverse-sweep table G holds the same rows
 // (RevStride<D>::S floats per cell).
-// Launch bound: 1024 threads (4 waves per SIMD, up to 128 VGPRs) for the
-// register variant without adaptive substeps (cells only in registers: ~90
-// VGPRs in 2D, ~120 in 3D); 768 (3 waves per SIMD, up to 168 VGPRs) for the
-// segmented variant and the adaptive register variant, whose trajectory takes
-// D x 50 VGPRs.
-template <int D, bool ADAPTIVE, int TS>
-constexpr int kBwdThreads = (TS > 0 && !ADAPTIVE) ? 1024 : 768;
+// Launch bound: 1024 threads (4 waves per SIMD, up to 128 VGPRs) where only
+// the cells are in registers (the register variant without adaptive substeps:
+// ~90 VGPRs in 2D, ~120 in 3D; the trail up to 64 steps: ~100 and ~122); 768
+// (3 waves per SIMD, up to 168 VGPRs) for the longer trail, the segmented
+// variant and the adaptive register variant, whose trajectory takes D x 50
+// VGPRs.
+template <bool ADAPTIVE, int BODY>
+constexpr int kBwdThreads = (BODY == kBodyTrail64 || (BODY == kBodyRegister && !ADAPTIVE)) ? 1024 : 768;
 
-template <int D, bool ADAPTIVE, bool LDS_A, int BINS, int TS>
-__global__ __launch_bounds__((kBwdThreads<D, ADAPTIVE, TS>)) void backward_kernel(
+template <int D, bool ADAPTIVE, bool LDS_A, int BINS, int BODY>
+__global__ __launch_bounds__((kBwdThreads<ADAPTIVE, BODY>)) void backward_kernel(
     int nP, int batched, int T, Cells g, int nC, int K, const float* __restrict__ points,
     const float* __restrict__ stage_points, const float* __restrict__ As,
     const float* __restrict__ Gs, Recover rec, const float* __restrict__ grad_out,
@@ -103,9 +108,9 @@ __global__ __launch_bounds__((kBwdThreads<D, ADAPTIVE, TS>)) void backward_kerne
     io.gout = k == K - 1 ? grad_out + (size_t)b * plane : lam + (size_t)b * plane;
     io.lam_out = k == 0 ? (grad_points ? grad_points + (size_t)b * plane : nullptr)
                         : lam + (size_t)b * plane;
-    const float delta = stage_delta<D, ADAPTIVE, TS>(rec, row, g);
+    const float delta = stage_delta<D, ADAPTIVE, BODY>(rec, row, T, g);
     L.begin(Ag, Gg, R, nC * RevStride<D>::S, &touched_cnt);
-    run_stage<D, ADAPTIVE, LDS_A, BINS, TS>(L, Ag, Gg, nP, T, g, io, moments + row * R, rec, row,
+    run_stage<D, ADAPTIVE, LDS_A, BINS, BODY>(L, Ag, Gg, nP, T, g, io, moments + row * R, rec, row,
                                             delta);
     // Every lane is done with this stage's tables before they are written out
     // (and, for the next stage, overwritten).
@@ -118,8 +123,8 @@ __global__ __launch_bounds__((kBwdThreads<D, ADAPTIVE, TS>)) void backward_kerne
 
 // Fused transform_data backward: one workgroup = one theta x one contiguous
 // range of output positions.
-template <int D, bool ADAPTIVE, bool LDS_A, int BINS, int TS>
-__global__ __launch_bounds__((kBwdThreads<D, ADAPTIVE, TS>)) void image_backward_kernel(
+template <int D, bool ADAPTIVE, bool LDS_A, int BINS, int BODY>
+__global__ __launch_bounds__((kBwdThreads<ADAPTIVE, BODY>)) void image_backward_kernel(
     ImageShape s, int T, Cells g, int nC, const float* __restrict__ axes,
     const float* __restrict__ final_points, const float* __restrict__ seed_grad,
     const float* __restrict__ As,
@@ -143,9 +148,9 @@ __global__ __launch_bounds__((kBwdThreads<D, ADAPTIVE, TS>)) void image_backward
   io.gout = grad_out + (size_t)b * s.C * s.nP;
   io.data = data + (size_t)b * s.C * s.plane_in;
   io.gdata = FloatScatter{grad_data ? grad_data + (size_t)b * s.C * s.plane_in : nullptr};
-  const float delta = stage_delta<D, ADAPTIVE, TS>(rec, (size_t)b, g);
+  const float delta = stage_delta<D, ADAPTIVE, BODY>(rec, (size_t)b, T, g);
   L.begin(Ag, Gg, R, nC * RevStride<D>::S, &touched_cnt);
-  run_stage<D, ADAPTIVE, LDS_A, BINS, TS>(L, Ag, Gg, s.nP, T, g, io, moments + (size_t)b * R, rec,
+  run_stage<D, ADAPTIVE, LDS_A, BINS, BODY>(L, Ag, Gg, s.nP, T, g, io, moments + (size_t)b * R, rec,
                                           (size_t)b, delta);
   const size_t part = (size_t)b * gridDim.x + w.part;
   L.end(partials + part * R, dense_parts + (size_t)b * ((gridDim.x + 63) / 64), w.part,
@@ -162,22 +167,24 @@ size_t stage_lds_bytes(int nC) {
   return lds;
 }
 
-template <int D, bool ADAPTIVE, bool LDS_A, int BINS, int TS>
+template <int D, bool ADAPTIVE, bool LDS_A, int BINS, int BODY>
 hipError_t go(const BackwardJob& j, const LaunchCfg& cfg, hipStream_t s) {
   const size_t lds = stage_lds_bytes<D, LDS_A, BINS>(j.geo.nC);
   const Cells g{j.geo.nx, j.geo.ny, j.geo.nz};
   const Recover rec{j.amp, adjoint_table_blocks(j.geo.nC),
-                    (float)std::pow((double)kRecoverGrowth, 1.0 / (double)j.T), j.edge};
+                    (float)std::pow((double)kRecoverGrowth,
+                                    1.0 / (double)(is_trail(BODY) ? kSeg : j.T)),
+                    j.edge};
   const dim3 grid((unsigned)cfg.chunks, (unsigned)j.n_batch), block((unsigned)cfg.block);
   if (j.image) {
-    auto kernel = image_backward_kernel<D, ADAPTIVE, LDS_A, BINS, TS>;
+    auto kernel = image_backward_kernel<D, ADAPTIVE, LDS_A, BINS, BODY>;
     hipError_t e = allow_lds(kernel, lds);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(kernel, grid, block, lds, s, *j.image, j.T, g, j.geo.nC, j.axes,
                        j.final_points, j.seed_grad, j.As, j.G, rec, j.data, j.grad_out, j.moments,
                        j.partials, j.dense_parts, j.grad_data);
   } else {
-    auto kernel = backward_kernel<D, ADAPTIVE, LDS_A, BINS, TS>;
+    auto kernel = backward_kernel<D, ADAPTIVE, LDS_A, BINS, BODY>;
     hipError_t e = allow_lds(kernel, lds);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(kernel, grid, block, lds, s, (int)j.nP, j.batched, j.T, g, j.geo.nC, j.K,
@@ -189,37 +196,40 @@ hipError_t go(const BackwardJob& j, const LaunchCfg& cfg, hipStream_t s) {
 
 template <int D>
 hipError_t dispatch(const BackwardJob& j, int adaptive, const LaunchCfg& cfg, hipStream_t s) {
-#define CPAB_GO(AD, LA, LB, TS) return go<D, AD, LA, LB, TS>(j, cfg, s)
-  // Register variant (the launch policy asks for it with full bins in 1D/2D,
-  // and without adaptive substeps in 3D, whose 150 VGPRs of trajectory leave
-  // no room for the adaptive step).
-  if (cfg.reg_steps == kRegSteps && j.T == kRegSteps) {
+#define CPAB_GO(AD, LA, LB, BODY) return go<D, AD, LA, LB, BODY>(j, cfg, s)
+  if (!adaptive) {
+    if (!cfg.trail && !cfg.reg_steps) CPAB_GO(false, false, kBinsCache, kBodySegmented);
     if constexpr (D <= 2) {
-      if (cfg.lds_bins) {
-        if (cfg.lds_rev) {
-          if (adaptive) CPAB_GO(true, false, kBinsFullRev, kRegSteps);
-          CPAB_GO(false, false, kBinsFullRev, kRegSteps);
-        }
-        if (adaptive) CPAB_GO(true, false, kBinsFull, kRegSteps);
-        CPAB_GO(false, false, kBinsFull, kRegSteps);
-      }
-    } else {
-      if (!adaptive) {
-        if (cfg.lds_bins) CPAB_GO(false, false, kBinsFull, kRegSteps);
-        CPAB_GO(false, false, kBinsCache, kRegSteps);
+      if (cfg.lds_rev) {
+        if (cfg.reg_steps) CPAB_GO(false, false, kBinsFullRev, kBodyRegister);
+        if (cfg.trail == 64) CPAB_GO(false, false, kBinsFullRev, kBodyTrail64);
+        CPAB_GO(false, false, kBinsFullRev, kBodyTrail104);
       }
     }
+    if (cfg.lds_bins) {
+      if (cfg.reg_steps) CPAB_GO(false, false, kBinsFull, kBodyRegister);
+      if (cfg.trail == 64) CPAB_GO(false, false, kBinsFull, kBodyTrail64);
+      CPAB_GO(false, false, kBinsFull, kBodyTrail104);
+    }
+    if constexpr (D == 3) {
+      if (cfg.reg_steps) CPAB_GO(false, false, kBinsCache, kBodyRegister);
+    }
+    if (cfg.trail == 64) CPAB_GO(false, false, kBinsCache, kBodyTrail64);
+    CPAB_GO(false, false, kBinsCache, kBodyTrail104);
   }
-  const int key = (adaptive ? 4 : 0) + (cfg.lds_table ? 2 : 0) + (cfg.lds_bins ? 1 : 0);
-  switch (key) {
-    case 0: CPAB_GO(false, false, kBinsCache, 0);
-    case 1: CPAB_GO(false, false, kBinsFull, 0);
-    case 2: CPAB_GO(false, true, kBinsCache, 0);
-    case 3: CPAB_GO(false, true, kBinsFull, 0);
-    case 4: CPAB_GO(true, false, kBinsCache, 0);
-    case 5: CPAB_GO(true, false, kBinsFull, 0);
-    case 6: CPAB_GO(true, true, kBinsCache, 0);
-    default: CPAB_GO(true, true, kBinsFull, 0);
+  // Adaptive substeps: the register variant for T == kRegSteps with full bins
+  // in 1D/2D (in 3D its 150 VGPRs of trajectory leave no room for the step).
+  if constexpr (D <= 2) {
+    if (cfg.reg_steps) {
+      if (cfg.lds_rev) CPAB_GO(true, false, kBinsFullRev, kBodyRegister);
+      CPAB_GO(true, false, kBinsFull, kBodyRegister);
+    }
+  }
+  switch ((cfg.lds_table ? 2 : 0) + (cfg.lds_bins ? 1 : 0)) {
+    case 0: CPAB_GO(true, false, kBinsCache, kBodySegmented);
+    case 1: CPAB_GO(true, false, kBinsFull, kBodySegmented);
+    case 2: CPAB_GO(true, true, kBinsCache, kBodySegmented);
+    default: CPAB_GO(true, true, kBinsFull, kBodySegmented);
   }
 #undef CPAB_GO
 }

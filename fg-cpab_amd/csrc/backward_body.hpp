@@ -512,14 +512,6 @@ __device__ __forceinline__ void segmented_run(P tab, const float* __restrict__ g
   }
 }
 
-template <int D, bool ADAPTIVE, int BINS, int MAXSEG = kMaxSeg, typename P, typename IO>
-__device__ __forceinline__ void segmented_body(P tab, const float* __restrict__ gtab, int nP, int T,
-                                               const Cells& g, const IO& io, float* bins,
-                                               int* keys, float* __restrict__ mom_b) {
-  segmented_run<D, ADAPTIVE, MAXSEG>(tab, gtab, nP, T, g, io,
-                                     FloatSink<BINS, Dim<D>::P>{bins, keys, mom_b});
-}
-
 // Register variant: T == TS known at compile time; each run's sums go to
 // `flush` (FloatSink: full LDS bins or, 3D, the LDS cell cache; or the
 // deterministic sink).  Without adaptive substeps every replay step is
@@ -658,6 +650,202 @@ __device__ __forceinline__ void register_body(P tab, PG gtab, int nP, const Cell
   if (kSpread && pend_on) flush(pend_c, pend);
 }
 
+// The cells of a whole trajectory in VGPRs, two 16-bit ids per register, for
+// any T <= CAP (64 or 104) known only at run time.  Registers are written and
+// read at a wave-uniform index (VGPR index mode: two scalar instructions and a
+// move), so the loops over the steps stay rolled and every T takes the same
+// code.  The first T % kSeg steps are group 0 (when there are any), the others
+// fill whole groups of kSeg steps.
+typedef uint32_t u32v4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32v16 __attribute__((ext_vector_type(16)));
+typedef uint32_t u32v32 __attribute__((ext_vector_type(32)));
+constexpr int kTrailWords = kSeg / 2;  // registers per group
+static_assert(kSeg == 8 && kMaxSteps <= 104, "Trail capacity");
+
+typedef float f32v8 __attribute__((ext_vector_type(8)));
+typedef float f32v16 __attribute__((ext_vector_type(16)));
+
+template <int CAP> struct Trail;
+template <> struct Trail<64> {
+  using Starts = f32v8;   // one float per group
+  u32v32 a;
+  __device__ __forceinline__ void clear() { a = 0; }
+  __device__ __forceinline__ void put(int i, uint32_t w) { a[i] = w; }
+  __device__ __forceinline__ uint32_t get(int i) const { return a[i]; }
+};
+template <> struct Trail<104> {
+  using Starts = f32v16;
+  u32v32 a;   // groups 0 .. 7
+  u32v16 b;   // groups 8 .. 11
+  u32v4 d;    // group 12 (T > 96)
+  __device__ __forceinline__ void clear() { a = 0; b = 0; d = 0; }
+  __device__ __forceinline__ void put(int i, uint32_t w) {
+    if (i < 32) a[i] = w;
+    else if (i < 48) b[i - 32] = w;
+    else d[i - 48] = w;
+  }
+  __device__ __forceinline__ uint32_t get(int i) const {
+    if (i < 32) return a[i];
+    if (i < 48) return b[i - 32];
+    return d[i - 48];
+  }
+};
+
+// register_body without adaptive substeps for any T <= CAP.  Each whole group's
+// start position is kept too, and phase 2 takes it up again at the group's end,
+// so a recovered position is at most kSeg steps of rounding away from the
+// replayed one (without that, the theta gradient of a [48, 48] field was three
+// times further from its 64-bit value), and a row need only keep the growth
+// bound over kSeg steps.
+// Bound by VALU issue and the latency of cell changes, as register_body.  One
+// midpoint pass and table reads only at cell changes, where the segmented body
+// makes two passes and reads an entry at every step: 16 thetas x 60,001 points,
+// [16, 16], T = 20: 118 -> 75 us; 2 x 400,000 points, [48, 48] (LDS cell
+// cache), T = 50: 701 -> 211 us.
+template <int D, int CAP, typename P, typename PG, typename IO, typename Sink>
+__device__ __forceinline__ void trail_body(P tab, PG gtab, int nP, int T, const Cells& g,
+                                           const IO& io, const Sink& flush, float delta) {
+  constexpr int PP = Dim<D>::P;
+  constexpr bool kSpread = D <= 2 && Sink::kSpread;   // see register_body
+  const float h = 1.0f / (float)T;
+  const float hh = h * 0.5f;
+  const int head = T % kSeg, groups = T / kSeg;
+  const int word0 = head ? kTrailWords : 0;   // first whole group's register
+  float pend[PP];
+#pragma unroll
+  for (int k = 0; k < PP; ++k) pend[k] = 0.0f;
+  int pend_c = 0;
+  bool pend_on = false;
+  int lo, hi;
+  wg_range(nP, lo, hi);
+  for (int base = lo; base < hi; base += blockDim.x) {
+    const int pi0 = base + (int)threadIdx.x;
+    const bool valid = pi0 < hi;
+    const int pi = valid ? pi0 : hi - 1;
+    float p[D];
+    io.start(pi, p);
+    float lam[D];
+    io.seed(pi, valid, lam);
+
+    // Phase 1: the midpoint trajectory; the cells to the trail.
+    Trail<CAP> trail;
+    trail.clear();
+    typename Trail<CAP>::Starts starts[D];
+#pragma unroll
+    for (int k = 0; k < D; ++k) starts[k] = 0.0f;
+    int c = 0;
+    auto phase1 = [&](auto inside) {
+      constexpr bool kInside = decltype(inside)::value;
+      auto look = [&]() {
+        if constexpr (kInside) return lookup_inside<D>(p, g);
+        else return lookup<D>(p, g);
+      };
+      c = look();
+      Aff<D> A = fetch<D>(tab, c);
+      auto step = [&]() {
+        const int cn = look();
+        // Divergent branch, skipped (exec = 0) when no lane changed cell.
+        if (__builtin_expect(cn != c, 0)) A = fetch<D>(tab, cn);
+        c = cn;
+        midpoint(A, p, h, hh);
+        return (uint32_t)cn;
+      };
+      uint32_t pair = 0;
+#pragma unroll 1
+      for (int t = 0; t < head; ++t) {
+        pair = (t & 1) ? pair | (step() << 16) : step();
+        trail.put(t >> 1, pair);
+      }
+#pragma unroll 1
+      for (int q = 0; q < groups; ++q) {
+        if constexpr (kSpread) {
+          if (q < PP) {
+            const float v = stack_pop(pend);
+            if (pend_on) flush.add1(pend_c, q, v);
+          }
+        }
+#pragma unroll
+        for (int k = 0; k < D; ++k) starts[k][q] = p[k];
+        uint32_t w[kTrailWords];
+#pragma unroll
+        for (int k = 0; k < kTrailWords; ++k) {
+          w[k] = step();
+          w[k] |= step() << 16;
+        }
+#pragma unroll
+        for (int k = 0; k < kTrailWords; ++k) trail.put(word0 + kTrailWords * q + k, w[k]);
+      }
+    };
+    if constexpr (D == 2) {
+      const float x0[1] = {p[0]}, y0[1] = {p[1]};
+      if (edge_safe(x0, y0, delta)) phase1(std::integral_constant<bool, true>{});
+      else phase1(std::integral_constant<bool, false>{});
+    } else {
+      phase1(std::integral_constant<bool, false>{});
+    }
+    if constexpr (kSpread) {
+      for (int k = groups; k < PP; ++k) {
+        const float v = stack_pop(pend);
+        if (pend_on) flush.add1(pend_c, k, v);
+      }
+    }
+
+    // Phase 2: reverse sweep from the last step's cell.
+    float m[PP];
+#pragma unroll
+    for (int k = 0; k < PP; ++k) m[k] = 0.0f;
+    Adj<D> G = fetch_adj<D>(gtab, c);
+    Inv<D> E = fetch_inv<D>(gtab, c);
+    auto back = [&](uint32_t cell) {
+      const int cn = (int)cell;
+      // Divergent branch, skipped where no lane changes cell; the next cell's
+      // entry is read before the finished cell's sums are added (LDS operations
+      // retire in order).
+      if (__builtin_expect(cn != c, 0)) {
+        G = fetch_adj<D>(gtab, cn);
+        E = fetch_inv<D>(gtab, cn);
+        if (valid) flush(c, m);
+#pragma unroll
+        for (int k = 0; k < PP; ++k) m[k] = 0.0f;
+      }
+      c = cn;
+      step_back<D>(E, p);  // p = position at this step
+      adjoint(G, p, m, lam);
+      // The lambda update reads G: finish it before a branch that reloads G.
+      pin(lam);
+    };
+#pragma unroll 1
+    for (int q = groups - 1; q >= 0; --q) {
+      uint32_t w[kTrailWords];
+#pragma unroll
+      for (int k = 0; k < kTrailWords; ++k) w[k] = trail.get(word0 + kTrailWords * q + k);
+#pragma unroll
+      for (int k = kTrailWords - 1; k >= 0; --k) {
+        back(w[k] >> 16);
+        back(w[k] & 0xffffu);
+      }
+#pragma unroll
+      for (int k = 0; k < D; ++k) p[k] = starts[k][q];
+    }
+#pragma unroll 1
+    for (int t = head - 1; t >= 0; --t) {
+      const uint32_t w = trail.get(t >> 1);
+      back((t & 1) ? w >> 16 : w & 0xffffu);
+    }
+    if constexpr (kSpread) {
+      wave_run_sums<PP>(valid, c, m, pend, pend_on);
+      pend_c = c;
+    } else {
+      float r[PP];
+      bool on;
+      wave_run_sums<PP>(valid, c, m, r, on);
+      if (on) flush(c, r);
+    }
+    io.finish(pi, valid, lam);
+  }
+  if (kSpread && pend_on) flush(pend_c, pend);
+}
+
 // LDS layout of a backward workgroup: [A table (LDS_A)] then either the full
 // bins (R floats) or the cache (kCacheSlots keys, then kCacheSlots * PP floats).
 template <int D, bool LDS_A, int BINS>
@@ -754,6 +942,12 @@ __device__ __forceinline__ bool recover_ok(const float* __restrict__ amp_row, in
   return __builtin_amdgcn_readfirstlane(a <= amp_max ? 1 : 0) != 0;
 }
 
+// What a backward kernel runs per trajectory: the segmented body (any T), the
+// register body (T == kRegSteps, unrolled), or the trail body for T <= 64 or
+// T <= 104.
+enum Body { kBodySegmented, kBodyRegister, kBodyTrail64, kBodyTrail104 };
+constexpr bool is_trail(int body) { return body == kBodyTrail64 || body == kBodyTrail104; }
+
 // Row stability of the register variant: the per-row block maxima of ||M_c||_2
 // and the bound they are held to.
 struct Recover {
@@ -780,38 +974,44 @@ __device__ __forceinline__ float row_edge_delta(const EdgeAcc* __restrict__ part
 // The row's domain-edge bound for the register variant's replay (2D without
 // adaptive substeps and with bound parts), else +inf.  Called before the
 // stage's tables are staged, so that its loads overlap theirs.
-template <int D, bool ADAPTIVE, int TS>
-__device__ __forceinline__ float stage_delta(const Recover& rec, size_t row, const Cells& g) {
-  if constexpr (D == 2 && !ADAPTIVE && TS > 0) {
-    if (rec.edge) return row_edge_delta(rec.edge + row * rec.namp, rec.namp, TS, g.nx, g.ny);
+template <int D, bool ADAPTIVE, int BODY>
+__device__ __forceinline__ float stage_delta(const Recover& rec, size_t row, int T, const Cells& g) {
+  if constexpr (D == 2 && BODY != kBodySegmented && !ADAPTIVE) {
+    if (rec.edge) return row_edge_delta(rec.edge + row * rec.namp, rec.namp, T, g.nx, g.ny);
   }
   return INFINITY;
 }
 
-template <int D, bool ADAPTIVE, bool LDS_A, int BINS, int TS, typename IO>
+template <int D, bool ADAPTIVE, bool LDS_A, int BINS, int BODY, typename IO>
 __device__ __forceinline__ void run_stage(const StageLds<D, LDS_A, BINS>& L, const float* Ag,
                                           const float* Gg, int nP, int T, const Cells& g,
                                           const IO& io, float* __restrict__ mom_b,
                                           const Recover& rec, size_t row, float delta) {
-  if constexpr (TS > 0) {
-    if constexpr (!ADAPTIVE) {
-      // Rows whose inverse maps could amplify the recovered positions' rounding
-      // beyond kRecoverGrowth replay each segment from a checkpoint instead.
-      if (!recover_ok(rec.amp + row * rec.namp, rec.namp, rec.amp_max)) {
-        constexpr int kSegs = (TS + kSeg - 1) / kSeg;
-        if (LDS_A) segmented_body<D, false, BINS, kSegs>(as_lds(L.ldsA), Gg, nP, TS, g, io, L.bins, L.keys, mom_b);
-        else segmented_body<D, false, BINS, kSegs>(Ag, Gg, nP, TS, g, io, L.bins, L.keys, mom_b);
-        return;
-      }
+  const FloatSink<BINS, Dim<D>::P> sink{L.bins, L.keys, mom_b};
+  if constexpr (BODY != kBodySegmented && !ADAPTIVE) {
+    // Rows whose inverse maps could amplify the recovered positions' rounding
+    // beyond kRecoverGrowth replay each segment from a checkpoint instead.
+    if (!recover_ok(rec.amp + row * rec.namp, rec.namp, rec.amp_max)) {
+      constexpr int kSteps = BODY == kBodyRegister ? kRegSteps : BODY == kBodyTrail64 ? 64 : 104;
+      segmented_run<D, false, (kSteps + kSeg - 1) / kSeg>(
+          Ag, Gg, nP, BODY == kBodyRegister ? kRegSteps : T, g, io, sink);
+      return;
     }
-    const FloatSink<BINS, Dim<D>::P> sink{L.bins, L.keys, mom_b};
+  }
+  if constexpr (is_trail(BODY)) {
+    constexpr int CAP = BODY == kBodyTrail64 ? 64 : 104;
     if constexpr (BINS == kBinsFullRev)
-      register_body<D, ADAPTIVE, TS>(Ag, as_lds(L.ldsG), nP, g, io, sink, delta);
-    else if (LDS_A) register_body<D, ADAPTIVE, TS>(as_lds(L.ldsA), Gg, nP, g, io, sink, delta);
-    else register_body<D, ADAPTIVE, TS>(Ag, Gg, nP, g, io, sink, delta);
+      trail_body<D, CAP>(Ag, as_lds(L.ldsG), nP, T, g, io, sink, delta);
+    else
+      trail_body<D, CAP>(Ag, Gg, nP, T, g, io, sink, delta);
+  } else if constexpr (BODY == kBodyRegister) {
+    if constexpr (BINS == kBinsFullRev)
+      register_body<D, ADAPTIVE, kRegSteps>(Ag, as_lds(L.ldsG), nP, g, io, sink, delta);
+    else
+      register_body<D, ADAPTIVE, kRegSteps>(Ag, Gg, nP, g, io, sink, delta);
   } else {
-    if (LDS_A) segmented_body<D, ADAPTIVE, BINS>(as_lds(L.ldsA), Gg, nP, T, g, io, L.bins, L.keys, mom_b);
-    else segmented_body<D, ADAPTIVE, BINS>(Ag, Gg, nP, T, g, io, L.bins, L.keys, mom_b);
+    if (LDS_A) segmented_run<D, ADAPTIVE, kMaxSeg>(as_lds(L.ldsA), Gg, nP, T, g, io, sink);
+    else segmented_run<D, ADAPTIVE, kMaxSeg>(Ag, Gg, nP, T, g, io, sink);
   }
 }
 

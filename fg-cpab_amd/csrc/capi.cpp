@@ -146,9 +146,10 @@ int adj_stride(int ndim) { return ndim == 1 ? 4 : (ndim == 2 ? 12 : 24); }
 
 // Backward: full LDS bins when a theta's nC x ppc table fits in LDS, else the
 // hashed LDS cell cache (at most 104 KiB, 3D).  Register variant for T = 50
-// (cells, and with adaptive substeps positions, in VGPRs; one 1024-lane
-// workgroup per CU, 768 with adaptive substeps); otherwise the segmented
-// variant, with the affine table in LDS beside the bins when both fit.
+// and trail variant for other T (cells, and with adaptive substeps at T = 50
+// positions, in VGPRs; one workgroup per CU of 1024 lanes, or 768 for the
+// variants that need more registers); otherwise the segmented variant, with
+// the affine table in LDS beside the bins when both fit.
 // Returns false (message set) if the device's LDS holds neither.
 bool backward_cfg(const cpab::Geometry& g, int64_t nP, int64_t n_theta, int T, int adaptive,
                   cpab::LaunchCfg* out) {
@@ -163,9 +164,15 @@ bool backward_cfg(const cpab::Geometry& g, int64_t nP, int64_t n_theta, int T, i
          (long long)cache, dev.lds);
     return false;
   }
-  const bool reg = T == cpab::kRegSteps && g.nC <= 65535 &&
-                   (g.ndim <= 2 ? c.lds_bins != 0 : !adaptive);
-  c.reg_steps = reg ? cpab::kRegSteps : 0;
+  // 16-bit cell ids.  T == 50 takes the unrolled register body (its loop-free
+  // form is 3-5 % faster than the trail's in 2D, the same in 3D); other T, and
+  // 2D tables beyond LDS, the trail.
+  const bool packs = g.nC <= 65535;
+  const bool unrolled = packs && T == cpab::kRegSteps &&
+                        (g.ndim <= 2 ? c.lds_bins != 0 : !adaptive);
+  c.reg_steps = unrolled ? cpab::kRegSteps : 0;
+  c.trail = packs && !adaptive && !unrolled ? (T <= 64 ? 64 : 104) : 0;
+  const bool reg = unrolled || c.trail;
   // Register variant with full bins in 1D/2D: the reverse-sweep table joins the
   // bins in LDS when both fit, so the entry phase 2 reloads at every cell
   // change comes from LDS (C2 backward 176 -> 170 us, C1 19.5 -> 18.6 us).
@@ -176,7 +183,7 @@ bool backward_cfg(const cpab::Geometry& g, int64_t nP, int64_t n_theta, int T, i
   const int64_t lds = used + (c.lds_table ? table : 0);
   int wg_per_cu;
   if (reg) {
-    c.block = adaptive ? 768 : 1024;  // the kernel's launch bound
+    c.block = adaptive || c.trail == 104 ? 768 : 1024;  // the kernel's launch bound
     wg_per_cu = 1;
   } else {
     // 32 waves per CU as 512-lane workgroups, as many as LDS allows; the cache
@@ -711,7 +718,12 @@ int cpab_backward_noalloc(int ndim, int64_t nP, int64_t n_theta, int batched, in
     if (det ? !det_cfg(g, nP, n_theta, &cfg)
             : !backward_cfg(g, nP, n_theta, nstepsolver, adaptive, &cfg))
       return CPAB_ERR_DEVICE;
-    const int64_t need = backward_workspace(g, nP, n_theta, 1, cfg, det).total;
+    int64_t need = backward_workspace(g, nP, n_theta, 1, cfg, det).total;
+    // The limit for step counts without an unrolled variant is the segmented
+    // variant's shape (the largest), whichever body runs.
+    cpab::LaunchCfg seg;
+    if (!det && !cfg.reg_steps && backward_cfg(g, nP, n_theta, 0, 1, &seg))
+      need = std::max(need, backward_workspace(g, nP, n_theta, 1, seg).total);
     if (need > kScratchBytes)
       return fail(CPAB_ERR_INVALID,
                   "cpab_backward_noalloc: this problem needs %lld bytes of workspace, beyond the "

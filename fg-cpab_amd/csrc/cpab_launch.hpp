@@ -50,6 +50,7 @@ struct LaunchCfg {
   int lds_table;    // backward, segmented variant: stage the per-theta affine table in LDS
   int lds_bins;     // backward: accumulate moments in full LDS bins (per-workgroup partials)
   int lds_cache;    // backward: else accumulate in the hashed LDS cell cache
+  int trail;        // backward: the trail body for T <= 64 or T <= 104 (0 = another body)
   int reg_steps;    // backward: compile-time step count of the register variant (0 = segmented)
   int lds_rev;      // backward, register variant with full bins: the reverse-sweep table in LDS too
 };
