@@ -130,8 +130,7 @@ __global__ __launch_bounds__((kBwdThreads<ADAPTIVE, BODY>)) void image_backward_
     const float* __restrict__ As,
     const float* __restrict__ Gs, Recover rec, const float* __restrict__ data,
     const float* __restrict__ grad_out,
-    float* __restrict__ moments, float* __restrict__ partials, uint64_t* __restrict__ dense_parts,
-    float* __restrict__ grad_data) {
+    float* __restrict__ moments, float* __restrict__ partials, uint64_t* __restrict__ dense_parts) {
   extern __shared__ __align__(16) float lds[];
   __shared__ int touched_cnt;
   const WgSlot w = wg_slot();
@@ -147,7 +146,6 @@ __global__ __launch_bounds__((kBwdThreads<ADAPTIVE, BODY>)) void image_backward_
   io.sgrad = seed_grad ? seed_grad + (size_t)b * D * s.nP : nullptr;
   io.gout = grad_out + (size_t)b * s.C * s.nP;
   io.data = data + (size_t)b * s.C * s.plane_in;
-  io.gdata = FloatScatter{grad_data ? grad_data + (size_t)b * s.C * s.plane_in : nullptr};
   const float delta = stage_delta<D, ADAPTIVE, BODY>(rec, (size_t)b, T, g);
   L.begin(Ag, Gg, R, nC * RevStride<D>::S, &touched_cnt);
   run_stage<D, ADAPTIVE, LDS_A, BINS, BODY>(L, Ag, Gg, s.nP, T, g, io, moments + (size_t)b * R, rec,
@@ -178,14 +176,16 @@ hipError_t go(const BackwardJob& j, const LaunchCfg& cfg, hipStream_t s) {
   const dim3 grid((unsigned)cfg.chunks, (unsigned)j.n_batch), block((unsigned)cfg.block);
   if (j.image) {
     auto kernel = image_backward_kernel<D, ADAPTIVE, LDS_A, BINS, BODY>;
-    hipError_t e = allow_lds(kernel, lds);
+    static LdsAllowed allowed;
+    hipError_t e = allow_lds(reinterpret_cast<const void*>(kernel), lds, allowed);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(kernel, grid, block, lds, s, *j.image, j.T, g, j.geo.nC, j.axes,
                        j.final_points, j.seed_grad, j.As, j.G, rec, j.data, j.grad_out, j.moments,
-                       j.partials, j.dense_parts, j.grad_data);
+                       j.partials, j.dense_parts);
   } else {
     auto kernel = backward_kernel<D, ADAPTIVE, LDS_A, BINS, BODY>;
-    hipError_t e = allow_lds(kernel, lds);
+    static LdsAllowed allowed;
+    hipError_t e = allow_lds(reinterpret_cast<const void*>(kernel), lds, allowed);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(kernel, grid, block, lds, s, (int)j.nP, j.batched, j.T, g, j.geo.nC, j.K,
                        j.points, j.stage_points, j.As, j.G, rec, j.grad_out, j.moments, j.partials,

@@ -297,7 +297,8 @@ hipError_t go_det(const BackwardJob& j, const LaunchCfg& cfg, hipStream_t s) {
   const dim3 grid((unsigned)cfg.chunks, (unsigned)j.n_batch), block((unsigned)kDetThreads<D>);
   if (j.image) {
     auto kernel = det_image_backward_kernel<D, ADAPTIVE, PASS, FULL, TS>;
-    hipError_t e = allow_lds(kernel, lds);
+    static LdsAllowed allowed;
+    hipError_t e = allow_lds(reinterpret_cast<const void*>(kernel), lds, allowed);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(kernel, grid, block, lds, s, *j.image, j.T, g, j.geo.nC, j.axes,
                        j.final_points, j.seed_grad, j.As, j.G, rec, j.data, j.grad_out,
@@ -305,7 +306,8 @@ hipError_t go_det(const BackwardJob& j, const LaunchCfg& cfg, hipStream_t s) {
                        j.det_gsums);
   } else {
     auto kernel = det_backward_kernel<D, ADAPTIVE, PASS, FULL, TS>;
-    hipError_t e = allow_lds(kernel, lds);
+    static LdsAllowed allowed;
+    hipError_t e = allow_lds(reinterpret_cast<const void*>(kernel), lds, allowed);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(kernel, grid, block, lds, s, (int)j.nP, j.batched, j.T, g, j.geo.nC, j.K,
                        j.points, j.stage_points, j.As, j.G, rec, j.grad_out, j.det_stat,

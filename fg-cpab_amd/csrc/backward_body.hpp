@@ -348,8 +348,8 @@ struct PlainIO {
 // (coalesced seed reads) and 3D in meshgrid order (lanes along coordinate 0:
 // fewer cells per wave than image order, strided seed reads).  Start points
 // come from the per-axis coordinate vectors either way.  GS: where the seed's
-// corner scatter adds grad_data (FloatScatter: float atomics).
-template <int D, typename GS = FloatScatter>
+// corner scatter adds grad_data (the deterministic pass; NoScatter otherwise).
+template <int D, typename GS = NoScatter>
 struct ImageIO {
   static constexpr bool kMeshOrder = D == 3;
   ImageShape s;
@@ -1013,13 +1013,6 @@ __device__ __forceinline__ void run_stage(const StageLds<D, LDS_A, BINS>& L, con
     if (LDS_A) segmented_run<D, ADAPTIVE, kMaxSeg>(as_lds(L.ldsA), Gg, nP, T, g, io, sink);
     else segmented_run<D, ADAPTIVE, kMaxSeg>(Ag, Gg, nP, T, g, io, sink);
   }
-}
-
-template <typename Kern>
-hipError_t allow_lds(Kern kernel, size_t lds) {
-  if (lds <= 65536) return hipSuccess;
-  return hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
-                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
 }
 
 }  // namespace

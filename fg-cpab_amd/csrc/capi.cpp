@@ -886,6 +886,10 @@ int cpab_transform_data_backward(int ndim, int64_t n_batch, int64_t n_channels,
   if (rc) return rc;
   if (grad_data) {
     rc = check_hip(cpab::launch_fill(grad_data, n_batch * n_channels * img.plane_in, 0.0f, s), who);
+    if (rc == CPAB_OK && !det)
+      rc = check_hip(cpab::launch_image_scatter(ndim, img, n_batch, final_points, grad_out,
+                                                grad_data, s),
+                     who);
     if (rc) return rc;
   }
   hipEvent_t ev = nullptr;
@@ -926,7 +930,7 @@ int cpab_transform_data_backward(int ndim, int64_t n_batch, int64_t n_channels,
   }
   rc = check_hip(cpab::launch_image_backward(g, img, n_batch, nstepsolver, adaptive, axes,
                                              final_points, seed_grad, As, G, amp, edge, data,
-                                             grad_out, moments, partials, dense, grad_data, cfg, s),
+                                             grad_out, moments, partials, dense, nullptr, cfg, s),
                  who);
   prof_end(timed, ev, "image_backward", s);
   if (rc) return rc;

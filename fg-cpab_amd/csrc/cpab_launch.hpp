@@ -4,6 +4,8 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <atomic>
+#include <mutex>
 #include "cpab_sample.hpp"
 
 namespace cpab {
@@ -54,6 +56,28 @@ struct LaunchCfg {
   int reg_steps;    // backward: compile-time step count of the register variant (0 = segmented)
   int lds_rev;      // backward, register variant with full bins: the reverse-sweep table in LDS too
 };
+
+// Lets a kernel use `lds` bytes of dynamic LDS (beyond the default 64 KiB).  The
+// attribute belongs to the kernel on a device; `LdsAllowed`, one per kernel,
+// holds the largest size set per device (setting it again on every launch costs
+// the host about a microsecond).
+struct LdsAllowed {
+  std::atomic<size_t> bytes[64] = {};
+  std::mutex mu;   // sizes are set in growing order
+};
+inline hipError_t allow_lds(const void* kernel, size_t lds, LdsAllowed& set) {
+  if (lds <= 65536) return hipSuccess;
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return e;
+  const bool known = dev >= 0 && dev < 64;
+  if (known && set.bytes[dev].load(std::memory_order_relaxed) >= lds) return hipSuccess;
+  std::lock_guard<std::mutex> lock(set.mu);
+  if (known && set.bytes[dev].load(std::memory_order_relaxed) >= lds) return hipSuccess;
+  e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  if (e == hipSuccess && known) set.bytes[dev].store(lds, std::memory_order_relaxed);
+  return e;
+}
 
 hipError_t launch_fill(float* dst, int64_t n, float value, hipStream_t s);
 hipError_t launch_affine(int64_t n_theta, int rows, int d, const float* theta,
@@ -147,6 +171,13 @@ hipError_t launch_image_backward(const Geometry& g, const ImageShape& img, int64
                                  unsigned long long* det_sums = nullptr,
                                  unsigned* det_flags = nullptr, const unsigned* det_gstat = nullptr,
                                  unsigned long long* det_gsums = nullptr);
+// grad_data [n_batch, C, *in] (zero before) of the image backward from the
+// final points [n_batch, ndim, prod(out)] (image order) and grad_out.
+// launch_image_backward itself adds to grad_data only in its deterministic
+// pass.
+hipError_t launch_image_scatter(int ndim, const ImageShape& img, int64_t n_batch,
+                                const float* final_points, const float* grad_out,
+                                float* grad_data, hipStream_t s);
 // Deterministic grad_data of the image backward: det_gstat [n_batch] (zero
 // before) gets each batch row's largest finite |scatter contribution| from the
 // final points and grad_out; det pass 2 of launch_image_backward then adds the

@@ -253,9 +253,13 @@ __device__ __forceinline__ void blend_grad(const float* c, const Axis& ax, const
 // plane (the deterministic backward brings its own sink with the same add()).
 struct FloatScatter {
   float* __restrict__ p;
-  __device__ __forceinline__ bool on() const { return p != nullptr; }
-  __device__ __forceinline__ FloatScatter channel(int64_t off) const { return {p + off}; }
   __device__ __forceinline__ void add(int i, float v) const { add_at(p, i, v); }
+};
+// No scatter (the default image backward, whose grad_data has its own kernel).
+struct NoScatter {
+  __device__ __forceinline__ constexpr bool on() const { return false; }
+  __device__ __forceinline__ NoScatter channel(int64_t) const { return {}; }
+  __device__ __forceinline__ void add(int, float) const {}
 };
 
 // The corner scatter of grad_data: g times each corner's weight added into gd
@@ -288,12 +292,6 @@ __device__ __forceinline__ void scatter_to(const int* in, const G& gd, const Axi
       }
 }
 
-template <int ND>
-__device__ __forceinline__ void scatter(const int* in, float* __restrict__ gd, const Axis& ax,
-                                        const Axis& ay, const Axis& az, float g) {
-  scatter_to<ND>(in, FloatScatter{gd}, ax, ay, az, g);
-}
-
 // blend_grad into dxyz (may be null) and scatter into *gd (may be null).
 template <int ND, typename G>
 __device__ __forceinline__ void sample_grad_to(const int* in, const float* __restrict__ d,
@@ -305,14 +303,6 @@ __device__ __forceinline__ void sample_grad_to(const int* in, const float* __res
     blend_grad<ND>(c, ax, ay, az, g, dxyz);
   }
   if (gd) scatter_to<ND>(in, *gd, ax, ay, az, g);
-}
-
-template <int ND>
-__device__ __forceinline__ void sample_grad(const int* in, const float* __restrict__ d,
-                                            const Axis& ax, const Axis& ay, const Axis& az,
-                                            float g, float* dxyz, float* __restrict__ gd) {
-  const FloatScatter sink{gd};
-  sample_grad_to<ND>(in, d, ax, ay, az, g, dxyz, gd ? &sink : nullptr);
 }
 
 }  // namespace cpab

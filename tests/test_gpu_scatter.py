@@ -1,0 +1,54 @@
+"""The data gradient's LDS box: boxes at and beyond its capacity (10,000 positions),
+data of one row or column, partial tiles in both directions, the data gradient
+without the grid gradient, and the image backward's scatter at odd sizes,
+against the oracle within the bound of the other data-gradient tests."""
+import numpy as np
+import pytest
+import torch
+
+from cpab.pytorch._native import native
+from oracle import oracle as orc
+
+from helpers import cpab_for, scatter_magnitude, seeded_theta
+
+pytestmark = pytest.mark.gpu
+
+
+def _dev(a, cuda):
+    return torch.from_numpy(np.ascontiguousarray(a)).to(cuda)
+
+
+@pytest.mark.parametrize("ins,outs", [((100, 100), (32, 32)), ((100, 101), (33, 31)), ((1, 9), (40, 70)),
+                                      ((9, 1), (31, 33)), ((20, 20, 25), (32, 2, 32)),
+                                      ((20, 21, 25), (33, 3, 5)), ((1, 1, 4), (5, 2, 64))])
+def test_scatter_box_limits(cuda, ins, outs):
+    nd, B, C = len(ins), 2, 2
+    rng = np.random.default_rng(800 + ins[0])
+    data = rng.random((B, C, *ins)).astype(np.float32)
+    grid = rng.random((B, nd, int(np.prod(outs)))).astype(np.float32)
+    grid[:, :, :2] = [0.0, 1.0]            # the box of the first tile reaches both ends
+    gout = rng.standard_normal((B, C, *outs)).astype(np.float32)
+    gd = torch.full(data.shape, float("nan"), device=cuda)
+    native().interp_backward(nd, _dev(data, cuda), _dev(grid, cuda), outs, _dev(gout, cuda), None, gd)
+    _, rd = orc.interp_backward(nd, data, grid, outs, gout)
+    mag = scatter_magnitude(data.shape, grid, outs, gout)
+    err = np.abs(gd.cpu().numpy().astype(np.float64) - rd)
+    assert (err <= 1e-4 * mag + 1e-12).all(), float((err / (mag + 1e-30)).max())
+
+
+@pytest.mark.parametrize("tess,size", [([5, 4], (71, 45)), ([3, 2, 2], (19, 6, 37))])
+def test_image_scatter_odd_sizes(cuda, tess, size):
+    # theta and data gradients of the public call against the two-step
+    # composition (transform_grid of the meshgrid, then interpolate)
+    T = cpab_for(tess)
+    rng = np.random.default_rng(810)
+    data = _dev(rng.random((2, 3, *size)).astype(np.float32), cuda).requires_grad_()
+    theta = _dev(seeded_theta(T, 2, 0.5, 811), cuda).requires_grad_()
+    g = _dev(rng.standard_normal((2, 3, *size)).astype(np.float32), cuda)
+    got = torch.autograd.grad(T.transform_data(data, theta, list(size)), (data, theta), g)
+    grid = T.transform_grid(T.uniform_meshgrid(list(size)), theta)
+    ref = torch.autograd.grad(T.interpolate(data, grid, list(size)), (data, theta), g)
+    # the same contributions per element in another order: a few float32 ulps
+    # of the largest sums
+    for a, b in zip(got, ref):
+        assert (a - b).abs().max().item() <= 2e-5 * b.abs().max().item()
