@@ -159,8 +159,9 @@ template <int D, bool LDS_A, int BINS>
 size_t stage_lds_bytes(int nC) {
   const size_t R = (size_t)nC * Dim<D>::P;
   size_t lds = LDS_A ? R * sizeof(float) : 0;
-  if (full_bins(BINS)) lds += R * sizeof(float);
-  if (BINS == kBinsFullRev) lds += (((R + 3) & ~(size_t)3) - R + (size_t)nC * RevStride<D>::S) * sizeof(float);
+  if (full_bins(BINS)) lds += R * sizeof(BinT<BINS>);
+  if (rev_in_lds(BINS))
+    lds += (((R + 3) & ~(size_t)3) - R) * sizeof(BinT<BINS>) + (size_t)nC * RevStride<D>::S * sizeof(float);
   if (BINS == kBinsCache) lds += (size_t)kCacheSlots * (Dim<D>::P + 1) * sizeof(float);
   return lds;
 }
@@ -174,22 +175,29 @@ hipError_t go(const BackwardJob& j, const LaunchCfg& cfg, hipStream_t s) {
                                     1.0 / (double)(is_trail(BODY) ? kSeg : j.T)),
                     j.edge};
   const dim3 grid((unsigned)cfg.chunks, (unsigned)j.n_batch), block((unsigned)cfg.block);
+  // Doubles serve single transforms of point arrays, and those always (see Bins).
   if (j.image) {
-    auto kernel = image_backward_kernel<D, ADAPTIVE, LDS_A, BINS, BODY>;
-    static LdsAllowed allowed;
-    hipError_t e = allow_lds(reinterpret_cast<const void*>(kernel), lds, allowed);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(kernel, grid, block, lds, s, *j.image, j.T, g, j.geo.nC, j.axes,
-                       j.final_points, j.seed_grad, j.As, j.G, rec, j.data, j.grad_out, j.moments,
-                       j.partials, j.dense_parts);
+    if constexpr (bins64(BINS)) return hipErrorInvalidValue;
+    else {
+      auto kernel = image_backward_kernel<D, ADAPTIVE, LDS_A, BINS, BODY>;
+      static LdsAllowed allowed;
+      hipError_t e = allow_lds(reinterpret_cast<const void*>(kernel), lds, allowed);
+      if (e != hipSuccess) return e;
+      hipLaunchKernelGGL(kernel, grid, block, lds, s, *j.image, j.T, g, j.geo.nC, j.axes,
+                         j.final_points, j.seed_grad, j.As, j.G, rec, j.data, j.grad_out, j.moments,
+                         j.partials, j.dense_parts);
+    }
   } else {
-    auto kernel = backward_kernel<D, ADAPTIVE, LDS_A, BINS, BODY>;
-    static LdsAllowed allowed;
-    hipError_t e = allow_lds(reinterpret_cast<const void*>(kernel), lds, allowed);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(kernel, grid, block, lds, s, (int)j.nP, j.batched, j.T, g, j.geo.nC, j.K,
-                       j.points, j.stage_points, j.As, j.G, rec, j.grad_out, j.moments, j.partials,
-                       j.dense_parts, j.lam, j.grad_points);
+    if constexpr (BINS == kBinsRev) return hipErrorInvalidValue;
+    else {
+      auto kernel = backward_kernel<D, ADAPTIVE, LDS_A, BINS, BODY>;
+      static LdsAllowed allowed;
+      hipError_t e = allow_lds(reinterpret_cast<const void*>(kernel), lds, allowed);
+      if (e != hipSuccess) return e;
+      hipLaunchKernelGGL(kernel, grid, block, lds, s, (int)j.nP, j.batched, j.T, g, j.geo.nC, j.K,
+                         j.points, j.stage_points, j.As, j.G, rec, j.grad_out, j.moments,
+                         j.partials, j.dense_parts, j.lam, j.grad_points);
+    }
   }
   return hipGetLastError();
 }
@@ -197,20 +205,20 @@ hipError_t go(const BackwardJob& j, const LaunchCfg& cfg, hipStream_t s) {
 template <int D>
 hipError_t dispatch(const BackwardJob& j, int adaptive, const LaunchCfg& cfg, hipStream_t s) {
 #define CPAB_GO(AD, LA, LB, BODY) return go<D, AD, LA, LB, BODY>(j, cfg, s)
+#define CPAB_STEPS(LB)                                            \
+  do {                                                            \
+    if (cfg.reg_steps) CPAB_GO(false, false, LB, kBodyRegister);  \
+    if (cfg.trail == 64) CPAB_GO(false, false, LB, kBodyTrail64); \
+    CPAB_GO(false, false, LB, kBodyTrail104);                     \
+  } while (0)
   if (!adaptive) {
     if (!cfg.trail && !cfg.reg_steps) CPAB_GO(false, false, kBinsCache, kBodySegmented);
     if constexpr (D <= 2) {
-      if (cfg.lds_rev) {
-        if (cfg.reg_steps) CPAB_GO(false, false, kBinsFullRev, kBodyRegister);
-        if (cfg.trail == 64) CPAB_GO(false, false, kBinsFullRev, kBodyTrail64);
-        CPAB_GO(false, false, kBinsFullRev, kBodyTrail104);
-      }
+      if (cfg.lds_rev && cfg.lds_bins64) CPAB_STEPS(kBinsRev64);
+      if (cfg.lds_rev) CPAB_STEPS(kBinsRev);
     }
-    if (cfg.lds_bins) {
-      if (cfg.reg_steps) CPAB_GO(false, false, kBinsFull, kBodyRegister);
-      if (cfg.trail == 64) CPAB_GO(false, false, kBinsFull, kBodyTrail64);
-      CPAB_GO(false, false, kBinsFull, kBodyTrail104);
-    }
+    if (cfg.lds_bins64) CPAB_STEPS(kBinsFull64);
+    if (cfg.lds_bins) CPAB_STEPS(kBinsFull);
     if constexpr (D == 3) {
       if (cfg.reg_steps) CPAB_GO(false, false, kBinsCache, kBodyRegister);
     }
@@ -221,7 +229,9 @@ hipError_t dispatch(const BackwardJob& j, int adaptive, const LaunchCfg& cfg, hi
   // in 1D/2D (in 3D its 150 VGPRs of trajectory leave no room for the step).
   if constexpr (D <= 2) {
     if (cfg.reg_steps) {
-      if (cfg.lds_rev) CPAB_GO(true, false, kBinsFullRev, kBodyRegister);
+      if (cfg.lds_rev && cfg.lds_bins64) CPAB_GO(true, false, kBinsRev64, kBodyRegister);
+      if (cfg.lds_rev) CPAB_GO(true, false, kBinsRev, kBodyRegister);
+      if (cfg.lds_bins64) CPAB_GO(true, false, kBinsFull64, kBodyRegister);
       CPAB_GO(true, false, kBinsFull, kBodyRegister);
     }
   }
@@ -231,6 +241,7 @@ hipError_t dispatch(const BackwardJob& j, int adaptive, const LaunchCfg& cfg, hi
     case 2: CPAB_GO(true, true, kBinsCache, kBodySegmented);
     default: CPAB_GO(true, true, kBinsFull, kBodySegmented);
   }
+#undef CPAB_STEPS
 #undef CPAB_GO
 }
 

@@ -7,6 +7,7 @@
 #include <hip/hip_runtime.h>
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 #include "cpab_device.hpp"
 #include "cpab_launch.hpp"
 #include "cpab_sample.hpp"
@@ -190,18 +191,33 @@ __device__ __forceinline__ float stack_pop(float (&a)[N]) {
   return v;
 }
 
-// Where the backward keeps its per-cell sums: full LDS bins, the hashed LDS
-// cell cache, or full bins with the reverse-sweep table (G and the inverse
-// one-step maps) staged in LDS beside them (register variant, 1D/2D).
-enum Bins { kBinsFull = 1, kBinsCache = 2, kBinsFullRev = 3 };
-constexpr bool full_bins(int b) { return b == kBinsFull || b == kBinsFullRev; }
+// Where the backward keeps its per-cell sums: full LDS bins in float or in
+// double (and, with kBinsRev*, the reverse-sweep table, G and the inverse
+// one-step maps, staged in LDS beside them), or the hashed LDS cell cache.
+//
+// Double because of the LDS atomic unit, not of the rounding: ds_add_f64 takes
+// 9 to 17 cycles for a whole wave, ds_add_f32 3 cycles per active lane (6 for
+// one or two lanes, 194 for 64), and every trajectory ends in a flush of all
+// lanes at once (C2 backward 163 -> 154 us; 16 thetas x 60,001 points, T = 20:
+// 75 -> 57 us; 8 x 40,000 points, [5, 5, 5]: 86 -> 76 us).  Single transforms of
+// point arrays take it where it fits.  The image backward, and chains, whose
+// points are mostly pixel grids, keep float: there wave_run_sums leaves few
+// lanes to flush and the conversions cost more than they save (16 x 512^2,
+// [12, 12]: 289 -> 298 us in double; 8 stages over 512^2 180 -> 185 us, though
+// over random points 199 -> 171 us).
+enum Bins { kBinsFull = 1, kBinsCache = 2, kBinsRev = 3, kBinsFull64 = 4, kBinsRev64 = 5 };
+constexpr bool full_bins(int b) { return b != kBinsCache; }
+constexpr bool rev_in_lds(int b) { return b == kBinsRev || b == kBinsRev64; }
+constexpr bool bins64(int b) { return b == kBinsFull64 || b == kBinsRev64; }
+template <int BINS>
+using BinT = std::conditional_t<bins64(BINS), double, float>;
 
-template <int P>
-__device__ __forceinline__ void flush_lds(float* bins, int c, const float (&m)[P]) {
-  float* q = bins + P * c;
+template <int P, typename V>
+__device__ __forceinline__ void flush_lds(V* bins, int c, const float (&m)[P]) {
+  V* q = bins + P * c;
 #pragma unroll
   for (int k = 0; k < P; ++k)
-    __hip_atomic_fetch_add(q + k, m[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    __hip_atomic_fetch_add(q + k, (V)m[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
 // Sums of a converged wave's last flush, pre-added per run of lanes with the
@@ -411,15 +427,16 @@ struct ImageIO {
 template <int BINS, int PP>
 struct FloatSink {
   static constexpr bool kSpread = full_bins(BINS);
-  float* bins;
+  BinT<BINS>* bins;
   int* keys;
   float* __restrict__ mom;
   __device__ __forceinline__ void operator()(int c, const float (&m)[PP]) const {
-    if (full_bins(BINS)) flush_lds<PP>(bins, c, m);
+    if constexpr (full_bins(BINS)) flush_lds<PP>(bins, c, m);
     else flush_cache<PP>(keys, bins, mom, c, m);
   }
   __device__ __forceinline__ void add1(int c, int k, float v) const {
-    __hip_atomic_fetch_add(bins + PP * c + k, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    __hip_atomic_fetch_add(bins + PP * c + k, (BinT<BINS>)v, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_WORKGROUP);
   }
 };
 
@@ -852,14 +869,14 @@ template <int D, bool LDS_A, int BINS>
 struct StageLds {
   float* ldsA;
   int* keys;
-  float* bins;
-  float* ldsG;   // kBinsFullRev: the reverse-sweep table after the bins
+  BinT<BINS>* bins;
+  float* ldsG;   // kBinsRev*: the reverse-sweep table after the bins
   __device__ __forceinline__ StageLds(float* lds, int R) {
     ldsA = lds;
     float* after_a = lds + (LDS_A ? R : 0);
     keys = reinterpret_cast<int*>(after_a);
-    bins = BINS == kBinsCache ? after_a + kCacheSlots : after_a;
-    ldsG = bins + ((R + 3) & ~3);   // 16-byte aligned
+    bins = reinterpret_cast<BinT<BINS>*>(BINS == kBinsCache ? after_a + kCacheSlots : after_a);
+    ldsG = reinterpret_cast<float*>(bins + ((R + 3) & ~3));   // 16-byte aligned
   }
   // Stage the tables, clear the bins / cache (and the touched-cell counter).
   __device__ __forceinline__ void begin(const float* __restrict__ Ag, const float* __restrict__ Gg,
@@ -870,7 +887,7 @@ struct StageLds {
       float2* d2 = reinterpret_cast<float2*>(ldsA);
       for (int i = threadIdx.x; i < R / 2; i += blockDim.x) d2[i] = s2[i];
     }
-    if (BINS == kBinsFullRev) {
+    if (rev_in_lds(BINS)) {
       // nG floats, a multiple of 4 (RevStride); the table and the LDS copy are
       // 16-byte aligned.
       const float4* s4 = reinterpret_cast<const float4*>(Gg);
@@ -878,11 +895,11 @@ struct StageLds {
       for (int i = threadIdx.x; i < nG / 4; i += blockDim.x) d4[i] = s4[i];
     }
     if (full_bins(BINS)) {
-      for (int i = threadIdx.x; i < R; i += blockDim.x) bins[i] = 0.0f;
+      for (int i = threadIdx.x; i < R; i += blockDim.x) bins[i] = 0;
       if (threadIdx.x == 0) *touched_cnt = 0;
     } else {
       for (int i = threadIdx.x; i < kCacheSlots; i += blockDim.x) keys[i] = -1;
-      for (int i = threadIdx.x; i < kCacheSlots * PP; i += blockDim.x) bins[i] = 0.0f;
+      for (int i = threadIdx.x; i < kCacheSlots * PP; i += blockDim.x) bins[i] = 0;
     }
     __syncthreads();
   }
@@ -899,7 +916,7 @@ struct StageLds {
       auto cell_touched = [&](int i) {
         bool t = false;
 #pragma unroll
-        for (int k = 0; k < PP; ++k) t |= bins[i * PP + k] != 0.0f;
+        for (int k = 0; k < PP; ++k) t |= bins[i * PP + k] != 0;
         return t;
       };
       int cnt = 0;
@@ -908,7 +925,7 @@ struct StageLds {
       __syncthreads();
       const bool dense = 4 * *touched_cnt >= nC;
       if (dense) {
-        for (int i = threadIdx.x; i < nC * PP; i += blockDim.x) partial[i] = bins[i];
+        for (int i = threadIdx.x; i < nC * PP; i += blockDim.x) partial[i] = (float)bins[i];
         if (threadIdx.x == 0)
           __hip_atomic_fetch_or(dense_parts + part / 64, 1ull << (part & 63), __ATOMIC_RELAXED,
                                 __HIP_MEMORY_SCOPE_AGENT);
@@ -916,14 +933,14 @@ struct StageLds {
         for (int i = threadIdx.x; i < nC; i += blockDim.x) {
           if (!cell_touched(i)) continue;
 #pragma unroll
-          for (int k = 0; k < PP; ++k) unsafeAtomicAdd(mom_b + (size_t)i * PP + k, bins[i * PP + k]);
+          for (int k = 0; k < PP; ++k) unsafeAtomicAdd(mom_b + (size_t)i * PP + k, (float)bins[i * PP + k]);
         }
       }
     } else {
       for (int i = threadIdx.x; i < kCacheSlots * PP; i += blockDim.x) {
         const int slot = i / PP;
         const int c = keys[slot];
-        if (c >= 0) unsafeAtomicAdd(mom_b + (size_t)PP * c + (i - slot * PP), bins[i]);
+        if (c >= 0) unsafeAtomicAdd(mom_b + (size_t)PP * c + (i - slot * PP), (float)bins[i]);
       }
     }
   }
@@ -1000,12 +1017,12 @@ __device__ __forceinline__ void run_stage(const StageLds<D, LDS_A, BINS>& L, con
   }
   if constexpr (is_trail(BODY)) {
     constexpr int CAP = BODY == kBodyTrail64 ? 64 : 104;
-    if constexpr (BINS == kBinsFullRev)
+    if constexpr (rev_in_lds(BINS))
       trail_body<D, CAP>(Ag, as_lds(L.ldsG), nP, T, g, io, sink, delta);
     else
       trail_body<D, CAP>(Ag, Gg, nP, T, g, io, sink, delta);
   } else if constexpr (BODY == kBodyRegister) {
-    if constexpr (BINS == kBinsFullRev)
+    if constexpr (rev_in_lds(BINS))
       register_body<D, ADAPTIVE, kRegSteps>(Ag, as_lds(L.ldsG), nP, g, io, sink, delta);
     else
       register_body<D, ADAPTIVE, kRegSteps>(Ag, Gg, nP, g, io, sink, delta);

@@ -144,6 +144,10 @@ cpab::LaunchCfg forward_cfg(const cpab::Geometry& g, int64_t nP, int64_t n_theta
 // Floats per cell of the reverse-sweep table (cpab_device.hpp RevStride).
 int adj_stride(int ndim) { return ndim == 1 ? 4 : (ndim == 2 ? 12 : 24); }
 
+// What a backward runs over: one transform of a point array, a chain of them, or
+// an image.
+enum class Work { kPoints, kChain, kImage };
+
 // Backward: full LDS bins when a theta's nC x ppc table fits in LDS, else the
 // hashed LDS cell cache (at most 104 KiB, 3D).  Register variant for T = 50
 // and trail variant for other T (cells, and with adaptive substeps at T = 50
@@ -152,7 +156,7 @@ int adj_stride(int ndim) { return ndim == 1 ? 4 : (ndim == 2 ? 12 : 24); }
 // the affine table in LDS beside the bins when both fit.
 // Returns false (message set) if the device's LDS holds neither.
 bool backward_cfg(const cpab::Geometry& g, int64_t nP, int64_t n_theta, int T, int adaptive,
-                  cpab::LaunchCfg* out) {
+                  cpab::LaunchCfg* out, Work work = Work::kPoints) {
   const DeviceInfo dev = device_info();
   const int64_t table = (int64_t)g.nC * g.ppc() * 4;
   const int64_t cache = (int64_t)cpab::kCacheSlots * (g.ppc() + 1) * 4;
@@ -173,11 +177,18 @@ bool backward_cfg(const cpab::Geometry& g, int64_t nP, int64_t n_theta, int T, i
   c.reg_steps = unrolled ? cpab::kRegSteps : 0;
   c.trail = packs && !adaptive && !unrolled ? (T <= 64 ? 64 : 104) : 0;
   const bool reg = unrolled || c.trail;
-  // Register variant with full bins in 1D/2D: the reverse-sweep table joins the
-  // bins in LDS when both fit, so the entry phase 2 reloads at every cell
-  // change comes from LDS (C2 backward 176 -> 170 us, C1 19.5 -> 18.6 us).
-  const int64_t rev = (int64_t)g.nC * adj_stride(g.ndim) * 4 + 16;
-  c.lds_rev = (reg && g.ndim <= 2 && c.lds_bins && table + rev <= dev.lds) ? 1 : 0;
+  // Register and trail variants with full bins: bins of doubles when they fit
+  // and the work takes them (backward_body.hpp, Bins), and in 1D/2D the
+  // reverse-sweep table beside the bins when that fits too, so the entry phase
+  // 2 reloads at every cell change comes from LDS (C2 backward 176 -> 170 us).
+  // A chain restages each stage's table: measured slower than L2 reads (C5
+  // backward 185 -> 190 us).
+  const int64_t rev = (int64_t)g.nC * adj_stride(g.ndim) * 4 + 32;
+  const int64_t budget = dev.lds - 512;   // the kernel's own few words
+  c.lds_bins64 = (reg && c.lds_bins && work == Work::kPoints && 2 * table <= budget) ? 1 : 0;
+  c.lds_rev = (reg && c.lds_bins && work != Work::kChain &&
+               (work == Work::kImage || c.lds_bins64) && g.ndim <= 2 &&
+               (c.lds_bins64 ? 2 : 1) * table + rev <= budget) ? 1 : 0;
   const int64_t used = c.lds_bins ? table : cache;
   c.lds_table = (!reg && used + table <= dev.lds) ? 1 : 0;
   const int64_t lds = used + (c.lds_table ? table : 0);
@@ -441,11 +452,10 @@ int backward_impl(const char* who, int ndim, int64_t nP, int64_t n_batch, int ba
   if (K > 1) CPAB_REQUIRE(stage_points);
   const bool det = t_deterministic != 0;
   cpab::LaunchCfg cfg;
-  if (det ? !det_cfg(g, nP, n_batch, &cfg) : !backward_cfg(g, nP, n_batch, nstepsolver, adaptive, &cfg))
+  if (det ? !det_cfg(g, nP, n_batch, &cfg)
+          : !backward_cfg(g, nP, n_batch, nstepsolver, adaptive, &cfg,
+                          K > 1 ? Work::kChain : Work::kPoints))
     return CPAB_ERR_DEVICE;
-  // A chain restages each stage's table: measured slower than L2 reads (C5
-  // backward 185 -> 190 us), so chains keep the reverse-sweep table in HBM.
-  if (K > 1) cfg.lds_rev = 0;
   const BackwardWorkspace w = backward_workspace(g, nP, n_batch, K, cfg, det);
   if (workspace == nullptr || workspace_bytes < w.total)
     return fail(CPAB_ERR_INVALID, "workspace too small: need %lld bytes, got %lld",
@@ -858,7 +868,7 @@ int cpab_transform_data_backward(int ndim, int64_t n_batch, int64_t n_channels,
   const bool det = t_deterministic != 0;
   cpab::LaunchCfg cfg;
   if (det ? !det_cfg(g, img.nP, n_batch, &cfg)
-          : !backward_cfg(g, img.nP, n_batch, nstepsolver, adaptive, &cfg))
+          : !backward_cfg(g, img.nP, n_batch, nstepsolver, adaptive, &cfg, Work::kImage))
     return CPAB_ERR_DEVICE;
   const BackwardWorkspace w = backward_workspace(g, img.nP, n_batch, 1, cfg, det);
   // the deterministic grad_data's sums follow

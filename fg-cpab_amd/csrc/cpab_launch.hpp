@@ -54,7 +54,8 @@ struct LaunchCfg {
   int lds_cache;    // backward: else accumulate in the hashed LDS cell cache
   int trail;        // backward: the trail body for T <= 64 or T <= 104 (0 = another body)
   int reg_steps;    // backward: compile-time step count of the register variant (0 = segmented)
-  int lds_rev;      // backward, register variant with full bins: the reverse-sweep table in LDS too
+  int lds_bins64;   // backward, register and trail variants with full bins: bins of doubles
+  int lds_rev;      // and (1D/2D) the reverse-sweep table in LDS too
 };
 
 // Lets a kernel use `lds` bytes of dynamic LDS (beyond the default 64 KiB).  The

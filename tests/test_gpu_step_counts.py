@@ -23,7 +23,10 @@ def test_backward_step_counts(cuda, tess, nstep):
 
 @pytest.mark.parametrize("tess,nstep,n,scale", [([48, 48], 50, 9000, 0.5), ([48, 48], 66, 3000, 0.5),
                                                 ([10, 10, 10], 70, 3000, 0.5), ([20, 20], 20, 3000, 6.0),
-                                                ([50], 13, 3000, 10.0), ([4, 4, 4], 90, 2000, 6.0)])
+                                                ([50], 13, 3000, 10.0), ([4, 4, 4], 90, 2000, 6.0),
+                                                # bins of doubles without the reverse table, float bins
+                                                ([22, 22], 50, 9000, 0.5), ([32, 32], 50, 9000, 0.5),
+                                                ([32, 32], 30, 3000, 0.5), ([7, 7, 7], 50, 3000, 0.5)])
 def test_backward_step_counts_cache_and_strong(cuda, tess, nstep, n, scale):
     _check(tess, nstep, n, scale, cuda)
 
