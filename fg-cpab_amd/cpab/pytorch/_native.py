@@ -329,6 +329,27 @@ def profile_read(kernel):
     return ms.value, n.value
 
 
+BINDING_PATH = os.path.join(os.path.dirname(LIB_PATH), "_cpab_torch.so")
+_binding = None
+
+
+def torch_binding():
+    """The native autograd functions (``csrc/torch_binding.cpp``), loaded on first use."""
+    global _binding
+    if _binding is None:
+        load_library()
+        if not os.path.isfile(BINDING_PATH):
+            raise RuntimeError(f"_cpab_torch.so not found at {BINDING_PATH}; build it with "
+                               f"`make -C fg-cpab_amd/csrc` (or __graft_entry__.build())")
+        import importlib.util
+        import torch  # noqa: F401  (its libraries first)
+        spec = importlib.util.spec_from_file_location("_cpab_torch", BINDING_PATH)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        _binding = module
+    return _binding
+
+
 _native = None
 
 
