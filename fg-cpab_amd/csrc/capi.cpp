@@ -132,7 +132,10 @@ cpab::LaunchCfg forward_cfg(const cpab::Geometry& g, int64_t nP, int64_t n_theta
   cpab::LaunchCfg c{};
   // The kernels keep the current cell's map in registers and re-read the table
   // only when a lane changes cell, through L1/L2.
-  c.block = 512;
+  // Below two rounds of the chip's lanes smaller workgroups even out the last
+  // round (8 x 40,000 points in 3D: 24.6 us at 512 lanes, 22.5 at 256, 24.7 at
+  // 128; 8 x 50,021 in 2D, adaptive: 38.8, 36.4, 36.6).
+  c.block = nP * n_theta <= 2LL * dev.cus * 2048 ? 256 : 512;
   // Two rounds of resident workgroups (2048 lanes per CU) per CU.
   const int64_t want = (int64_t)dev.cus * (2048 / c.block) * 2;
   int64_t chunks = std::max<int64_t>(1, div_up(want, std::max<int64_t>(n_theta, 1)));
@@ -208,6 +211,46 @@ bool backward_cfg(const cpab::Geometry& g, int64_t nP, int64_t n_theta, int T, i
   c.chunks = (int)chunks;
   *out = c;
   return true;
+}
+
+// Lanes a workgroup of the register and trail variants has at least: enough
+// to clear, stage and write out its tables in a few dozen iterations.
+int64_t least_lanes(const cpab::Geometry& g, int most) {
+  const int64_t lanes = div_up((int64_t)g.nC * g.ppc() / 32, 64) * 64;
+  return std::min<int64_t>(std::max<int64_t>(lanes, 64), most);
+}
+
+// Spreads a register or trail backward's trajectories evenly: backward_cfg's
+// shape takes 1024-lane workgroups from a row's start, which leaves compute
+// units idle when a row is short (8 rows of 40,000 points: 160 workgroups of
+// 2048 points) and lanes idle in a last round.  Here a row is cut into
+// `chunks` nearly equal ranges, each covered in equal rounds by as many lanes
+// as that takes, with one to four workgroups for each compute unit (one at a
+// time fits, for large tables), whichever is estimated shortest: a round costs
+// a latency and its lanes (about a third and two thirds of a full round,
+// measured on short rows), a workgroup its tables.
+cpab::LaunchCfg spread_cfg(const cpab::Geometry& g, int64_t nP, int64_t n_theta,
+                           const cpab::LaunchCfg& base) {
+  if (!base.reg_steps && !base.trail) return base;
+  const int64_t cus = device_info().cus, n = std::max<int64_t>(n_theta, 1);
+  const int64_t most = std::max<int64_t>(1, div_up(nP, least_lanes(g, base.block)));
+  cpab::LaunchCfg best = base;
+  double least = 1e300;
+  for (int k = 1; k <= 4; ++k) {
+    const int64_t want = std::min(std::max<int64_t>(1, k * cus / n), most);
+    const int64_t per = div_up(nP, want), rounds = div_up(per, base.block);
+    const int64_t block = div_up(div_up(per, rounds), 64) * 64;
+    const int64_t chunks = div_up(nP, block * rounds);
+    const double tables = 0.25 + (double)g.nC * g.ppc() / 40000.0;
+    const double cost = (double)div_up(n * chunks, cus) *
+                        (tables + (double)rounds * (0.35 + 0.65 * (double)block / 1024.0));
+    if (cost < least * 0.98) {
+      least = cost;
+      best.chunks = (int)chunks;
+      best.block = (int)block;
+    }
+  }
+  return best;
 }
 
 hipStream_t as_stream(void* s) { return reinterpret_cast<hipStream_t>(s); }
@@ -398,10 +441,13 @@ int64_t workspace_size_impl(int ndim, int64_t nP, int64_t n_batch, int K, int nC
     if (!det_cfg(g, nP, n_batch, &det)) return 0;
     return backward_workspace(g, nP, n_batch, K, det, true).total;
   }
-  // Whichever variant runs (register or segmented) fits.
+  // Whichever variant runs (register, trail or segmented) fits, spread or not.
   cpab::LaunchCfg reg, seg;
   if (!backward_cfg(g, nP, n_batch, cpab::kRegSteps, 0, &reg) || !backward_cfg(g, nP, n_batch, 0, 1, &seg))
     return 0;
+  const int64_t wide = std::min<int64_t>(std::max<int64_t>(1, 4 * device_info().cus / n_batch),
+                                         div_up(nP, least_lanes(g, 768)));
+  reg.chunks = (int)std::max<int64_t>(reg.chunks, wide);
   return std::max(backward_workspace(g, nP, n_batch, K, reg).total,
                   backward_workspace(g, nP, n_batch, K, seg).total);
 }
@@ -456,7 +502,15 @@ int backward_impl(const char* who, int ndim, int64_t nP, int64_t n_batch, int ba
           : !backward_cfg(g, nP, n_batch, nstepsolver, adaptive, &cfg,
                           K > 1 ? Work::kChain : Work::kPoints))
     return CPAB_ERR_DEVICE;
-  const BackwardWorkspace w = backward_workspace(g, nP, n_batch, K, cfg, det);
+  BackwardWorkspace w = backward_workspace(g, nP, n_batch, K, cfg, det);
+  if (!det) {   // spread, where the caller's workspace has room for its partial tables
+    const cpab::LaunchCfg wide = spread_cfg(g, nP, n_batch, cfg);
+    const BackwardWorkspace ww = backward_workspace(g, nP, n_batch, K, wide);
+    if (ww.total <= workspace_bytes || ww.total <= w.total) {
+      cfg = wide;
+      w = ww;
+    }
+  }
   if (workspace == nullptr || workspace_bytes < w.total)
     return fail(CPAB_ERR_INVALID, "workspace too small: need %lld bytes, got %lld",
                 (long long)w.total, (long long)workspace_bytes);
@@ -870,7 +924,15 @@ int cpab_transform_data_backward(int ndim, int64_t n_batch, int64_t n_channels,
   if (det ? !det_cfg(g, img.nP, n_batch, &cfg)
           : !backward_cfg(g, img.nP, n_batch, nstepsolver, adaptive, &cfg, Work::kImage))
     return CPAB_ERR_DEVICE;
-  const BackwardWorkspace w = backward_workspace(g, img.nP, n_batch, 1, cfg, det);
+  BackwardWorkspace w = backward_workspace(g, img.nP, n_batch, 1, cfg, det);
+  if (!det) {   // as backward_impl
+    const cpab::LaunchCfg wide = spread_cfg(g, img.nP, n_batch, cfg);
+    const BackwardWorkspace ww = backward_workspace(g, img.nP, n_batch, 1, wide);
+    if (ww.total <= workspace_bytes || ww.total <= w.total) {
+      cfg = wide;
+      w = ww;
+    }
+  }
   // the deterministic grad_data's sums follow
   const bool det_data = det && grad_data != nullptr;
   const DataWorkspace dw = data_workspace(w.total, n_batch, n_channels, img.plane_in);
