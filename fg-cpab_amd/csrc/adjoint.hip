@@ -49,7 +49,7 @@
 //              HBM with global atomics.  Flushes that find no slot go
 //              straight to HBM.  The HBM table holds sums S; a separate pass
 //              forms the moments in place.
-// The cache takes at most 104 KiB of LDS (3D), within the 160 KiB a gfx950
+// The cache takes at most 154 KiB of LDS (2D), within the 160 KiB a gfx950
 // workgroup may use, so every tessellation runs one of the two.
 #include <hip/hip_runtime.h>
 #include <algorithm>
@@ -162,7 +162,7 @@ size_t stage_lds_bytes(int nC) {
   if (full_bins(BINS)) lds += R * sizeof(BinT<BINS>);
   if (rev_in_lds(BINS))
     lds += (((R + 3) & ~(size_t)3) - R) * sizeof(BinT<BINS>) + (size_t)nC * RevStride<D>::S * sizeof(float);
-  if (BINS == kBinsCache) lds += (size_t)kCacheSlots * (Dim<D>::P + 1) * sizeof(float);
+  if (BINS == kBinsCache) lds += cache_bytes(D);
   return lds;
 }
 

@@ -274,7 +274,8 @@ __device__ __forceinline__ void wave_run_sums(bool need, int c, const float (&m)
 template <int P>
 __device__ __forceinline__ void flush_cache(int* keys, float* vals, float* __restrict__ mom, int c,
                                             const float (&m)[P]) {
-  int slot = c & (kCacheSlots - 1);
+  constexpr unsigned S = kCacheSlots[P == 2 ? 1 : P == 6 ? 2 : 3];
+  unsigned slot = (unsigned)c % S;
   for (int probe = 0; probe < kCacheProbes; ++probe) {
     int k = __hip_atomic_load(keys + slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     if (k == -1) {
@@ -284,10 +285,10 @@ __device__ __forceinline__ void flush_cache(int* keys, float* vals, float* __res
       k = expected == -1 ? c : expected;
     }
     if (k == c) {
-      flush_lds<P>(vals, slot, m);
+      flush_lds<P>(vals, (int)slot, m);
       return;
     }
-    slot = (slot + 1) & (kCacheSlots - 1);
+    slot = slot + 1 == S ? 0 : slot + 1;
   }
 #pragma unroll
   for (int k = 0; k < P; ++k) unsafeAtomicAdd(mom + (size_t)P * c + k, m[k]);
@@ -864,7 +865,7 @@ __device__ __forceinline__ void trail_body(P tab, PG gtab, int nP, int T, const 
 }
 
 // LDS layout of a backward workgroup: [A table (LDS_A)] then either the full
-// bins (R floats) or the cache (kCacheSlots keys, then kCacheSlots * PP floats).
+// bins (R values) or the cache (kCacheSlots keys, then kCacheSlots * PP floats).
 template <int D, bool LDS_A, int BINS>
 struct StageLds {
   float* ldsA;
@@ -875,7 +876,7 @@ struct StageLds {
     ldsA = lds;
     float* after_a = lds + (LDS_A ? R : 0);
     keys = reinterpret_cast<int*>(after_a);
-    bins = reinterpret_cast<BinT<BINS>*>(BINS == kBinsCache ? after_a + kCacheSlots : after_a);
+    bins = reinterpret_cast<BinT<BINS>*>(BINS == kBinsCache ? after_a + kCacheSlots[D] : after_a);
     ldsG = reinterpret_cast<float*>(bins + ((R + 3) & ~3));   // 16-byte aligned
   }
   // Stage the tables, clear the bins / cache (and the touched-cell counter).
@@ -898,8 +899,8 @@ struct StageLds {
       for (int i = threadIdx.x; i < R; i += blockDim.x) bins[i] = 0;
       if (threadIdx.x == 0) *touched_cnt = 0;
     } else {
-      for (int i = threadIdx.x; i < kCacheSlots; i += blockDim.x) keys[i] = -1;
-      for (int i = threadIdx.x; i < kCacheSlots * PP; i += blockDim.x) bins[i] = 0;
+      for (int i = threadIdx.x; i < kCacheSlots[D]; i += blockDim.x) keys[i] = -1;
+      for (int i = threadIdx.x; i < kCacheSlots[D] * PP; i += blockDim.x) bins[i] = 0;
     }
     __syncthreads();
   }
@@ -937,7 +938,7 @@ struct StageLds {
         }
       }
     } else {
-      for (int i = threadIdx.x; i < kCacheSlots * PP; i += blockDim.x) {
+      for (int i = threadIdx.x; i < kCacheSlots[D] * PP; i += blockDim.x) {
         const int slot = i / PP;
         const int c = keys[slot];
         if (c >= 0) unsafeAtomicAdd(mom_b + (size_t)PP * c + (i - slot * PP), (float)bins[i]);

@@ -152,7 +152,7 @@ int adj_stride(int ndim) { return ndim == 1 ? 4 : (ndim == 2 ? 12 : 24); }
 enum class Work { kPoints, kChain, kImage };
 
 // Backward: full LDS bins when a theta's nC x ppc table fits in LDS, else the
-// hashed LDS cell cache (at most 104 KiB, 3D).  Register variant for T = 50
+// hashed LDS cell cache (at most 154 KiB, 2D).  Register variant for T = 50
 // and trail variant for other T (cells, and with adaptive substeps at T = 50
 // positions, in VGPRs; one workgroup per CU of 1024 lanes, or 768 for the
 // variants that need more registers); otherwise the segmented variant, with
@@ -162,7 +162,7 @@ bool backward_cfg(const cpab::Geometry& g, int64_t nP, int64_t n_theta, int T, i
                   cpab::LaunchCfg* out, Work work = Work::kPoints) {
   const DeviceInfo dev = device_info();
   const int64_t table = (int64_t)g.nC * g.ppc() * 4;
-  const int64_t cache = (int64_t)cpab::kCacheSlots * (g.ppc() + 1) * 4;
+  const int64_t cache = cpab::cache_bytes(g.ndim);
   cpab::LaunchCfg c{};
   c.lds_bins = table <= dev.lds ? 1 : 0;
   c.lds_cache = (!c.lds_bins && cache <= dev.lds) ? 1 : 0;
@@ -201,7 +201,7 @@ bool backward_cfg(const cpab::Geometry& g, int64_t nP, int64_t n_theta, int T, i
     wg_per_cu = 1;
   } else {
     // 32 waves per CU as 512-lane workgroups, as many as LDS allows; the cache
-    // variant runs one workgroup per CU (104 KiB of LDS in 3D): 12 waves.
+    // variant runs one workgroup per CU (104 to 154 KiB of LDS): 12 waves.
     c.block = c.lds_cache ? 768 : 512;
     wg_per_cu = (int)std::max<int64_t>(1, std::min<int64_t>(2048 / c.block, dev.lds / lds));
   }

@@ -40,9 +40,17 @@ constexpr int kRegSteps = 50;
 // reach 3e-5 .. 2.7e-4.
 constexpr float kRecoverGrowth = 16.0f;
 // Hashed LDS cell cache of the backward when the full moment table does not
-// fit in LDS: slots (a power of two) and linear-probe length.  3D: 2048 x 13
-// words = 104 KiB.
-constexpr int kCacheSlots = 2048;
+// fit in LDS: slots per ndim (a key and ppc floats each) and linear-probe
+// length.  2D: as many as fit (154 KB), because scattered points make a
+// workgroup touch most cells and a flush that finds no slot costs scattered
+// HBM atomics (2 x 400,000 points, [48, 48]: backward 199 us with 2048 slots,
+// 148 with 3072 of doubles, 139 with 5632 of floats; [64, 64]: 213, 169, 152).
+// 3D: 104 KB; 3072 slots were within 2 % (128^3 volume 308 -> 311 us, 2 x
+// 200,000 points at [9, 9, 9] 106 -> 104), 1536 of doubles slower (124).
+constexpr int kCacheSlots[4] = {0, 5632, 5632, 2048};
+constexpr int64_t cache_bytes(int ndim) {
+  return (int64_t)kCacheSlots[ndim] * 4 * (1 + ndim * (ndim + 1));
+}
 constexpr int kCacheProbes = 4;
 
 // Correctly rounded float exp / log / expm1: evaluated in double and rounded
