@@ -42,6 +42,21 @@ __global__ void affine_kernel(int64_t n_theta, int rows, int d, const float* __r
   As[i] = acc;
 }
 
+// acc + e[0].x * e[0].y + ... + e[n - 1].x * e[n - 1].y from LDS, one fma after
+// the other.
+__device__ __forceinline__ float add_in_order(const float2* e, int n, float acc) {
+  int k = 0;
+  for (; k + 4 <= n; k += 4) {
+    const float2 e0 = e[k], e1 = e[k + 1], e2 = e[k + 2], e3 = e[k + 3];
+    acc = fmaf(e0.x, e0.y, acc);
+    acc = fmaf(e1.x, e1.y, acc);
+    acc = fmaf(e2.x, e2.y, acc);
+    acc = fmaf(e3.x, e3.y, acc);
+  }
+  for (; k < n; ++k) acc = fmaf(e[k].x, e[k].y, acc);
+  return acc;
+}
+
 // grad[b, j] = sum_k B[row_k, j] * M[b, row_k] over the CSC column j of B,
 // added in ascending k with one fma per entry (a fixed order).  Each column is
 // served by kProjSeg lanes: they load its entries and gather the moments
@@ -99,19 +114,7 @@ __global__ __launch_bounds__(kProjThreads) void project_kernel(
       }
     }
     __syncthreads();
-    if (lane == 0 && base < k1) {
-      const int n = min(kProjCap, k1 - base);
-      int k = 0;
-      for (; k + 4 <= n; k += 4) {
-        const float2 e0 = stage[seg][k], e1 = stage[seg][k + 1];
-        const float2 e2 = stage[seg][k + 2], e3 = stage[seg][k + 3];
-        acc = fmaf(e0.x, e0.y, acc);
-        acc = fmaf(e1.x, e1.y, acc);
-        acc = fmaf(e2.x, e2.y, acc);
-        acc = fmaf(e3.x, e3.y, acc);
-      }
-      for (; k < n; ++k) acc = fmaf(stage[seg][k].x, stage[seg][k].y, acc);
-    }
+    if (lane == 0 && base < k1) acc = add_in_order(stage[seg], min(kProjCap, k1 - base), acc);
     __syncthreads();
   }
   if (live && lane == 0) grad[i] = acc;
@@ -469,26 +472,103 @@ __global__ void expm_kernel(int64_t n, float dT, const float* __restrict__ As,
 }
 
 // A = B theta and Trels = expm(dT A) in one launch.  A workgroup covers
-// kAffCells<D> consecutive (theta, cell) matrices: first one thread per row of
-// A forms it exactly as affine_kernel does (summed in ascending column order)
-// and stores it (coalesced) and into LDS; then one thread per cell
-// exponentiates its block as expm_kernel does and the results leave through
-// LDS, coalesced.  Both outputs equal the two-kernel sequence bit for bit.
-template <int D> constexpr int kAffCells = D == 1 ? 128 : (D == 2 ? 64 : 32);
+// kAffCells consecutive (theta, cell) matrices: first the rows of A are formed
+// in ascending column order, as affine_kernel does, and stored (coalesced) and
+// kept in LDS; then one thread per cell exponentiates its block as expm_kernel
+// does and the results leave through LDS, coalesced.  Both outputs equal the
+// two-kernel sequence bit for bit.
+//
+// LANES == 1: one thread per row and full waves of exponentials.  LANES == 8,
+// for up to kAffFew matrices: long rows take eight threads each (wide_row_sum).
+// One thread walking a long row (a field free at the boundary has 22 entries on
+// average and up to 42 at [8, 8], 72 at [3, 3, 3]) is a chain of memory round
+// trips, each lane of a wave in a cache line of its own, in few workgroups (32
+// for 2048 matrices).  Free fields, before and after: 8 thetas at [8, 8] 19.5 ->
+// 5.4 us, 16 of them 20.8 -> 5.8, 4 at [3, 3, 3] 33.9 -> 6.0.  The small
+// workgroups' exponentials fill an eighth of a wave, so short rows (1 to 3
+// entries, one thread each here too) pay 0.1 to 0.3 us up to 4096 matrices
+// (3.4 -> 3.7); beyond, several rounds of workgroups cost more (with eight
+// threads on short rows as well, 8192: 4.9 -> 7.0 us; 16,384: 3.7 -> 9.7).
+constexpr int kAffLanes = 8;
+constexpr int kAffFew = 4096;
+constexpr int kAffLong = 16;   // entries per row, on average, from which rows are long
+constexpr int kAffPer = 8;     // entries per thread and round
+template <int D, int LANES>
+constexpr int kAffCells = (D == 1 ? 256 : 384) / (D * (D + 1)) / LANES;
+template <int D, int LANES>
+constexpr int kAffThreads = kAffCells<D, LANES> * D * (D + 1) * LANES;
 
-template <int D>
-__global__ __launch_bounds__(kAffCells<D> * D * (D + 1)) void affine_expm_kernel(
+// The sum of the row's entries k0 .. k1 - 1 times theta, by LANES threads per
+// row (whole workgroup; the result is the first one's): they read the entries
+// in coalesced runs, gather their thetas together and stage both in LDS, and the
+// first adds them in order, as project_kernel does.
+template <int ROWS, int LANES>
+__device__ __forceinline__ float wide_row_sum(int k0, int k1, const float* __restrict__ th,
+                                              const int32_t* __restrict__ col_idx,
+                                              const float* __restrict__ vals) {
+  constexpr int CAP = LANES * kAffPer;
+  __shared__ float2 stage[ROWS][CAP + 1];   // a wave's rows start two banks apart
+  __shared__ int longest;
+  const int local = threadIdx.x / LANES, lane = threadIdx.x % LANES;
+  if (threadIdx.x == 0) longest = 0;
+  __syncthreads();
+  if (lane == 0) atomicMax(&longest, k1 - k0);
+  __syncthreads();
+  const int most = longest;                 // rounds: uniform over the workgroup
+  float acc = 0.0f;
+  for (int done = 0; done < most; done += CAP) {
+    const int from = k0 + done;
+    if (from < k1) {
+      // in-range loads (past the row's end its last entry, which is not added)
+      int idx[kAffPer];
+      float v[kAffPer], x[kAffPer];
+#pragma unroll
+      for (int u = 0; u < kAffPer; ++u) {
+        const int k = min(from + lane + u * LANES, k1 - 1);
+        idx[u] = col_idx[k];
+        v[u] = vals[k];
+      }
+#pragma unroll
+      for (int u = 0; u < kAffPer; ++u) x[u] = th[idx[u]];
+#pragma unroll
+      for (int u = 0; u < kAffPer; ++u) stage[local][lane + u * LANES] = make_float2(v[u], x[u]);
+    }
+    __syncthreads();
+    if (lane == 0 && from < k1) acc = add_in_order(stage[local], min(CAP, k1 - from), acc);
+    __syncthreads();
+  }
+  return acc;
+}
+
+template <int D, int LANES>
+__global__ __launch_bounds__((kAffThreads<D, LANES>)) void affine_expm_kernel(
     int64_t n_theta, int nC, int d, const float* __restrict__ theta,
     const int32_t* __restrict__ row_ptr, const int32_t* __restrict__ col_idx,
     const float* __restrict__ vals, float dT, float* __restrict__ As, float* __restrict__ Trels) {
   constexpr int P = D * (D + 1);
-  constexpr int CB = kAffCells<D>;
-  __shared__ float tile[CB * P];
+  constexpr int CB = kAffCells<D, LANES>;
+  constexpr int ROWS = CB * P;
+  __shared__ float tile[ROWS];
   const int64_t n = n_theta * nC * P;                  // rows of A in all
-  const int64_t base = (int64_t)blockIdx.x * CB * P;   // first row of this block
+  const int64_t base = (int64_t)blockIdx.x * ROWS;     // first row of this block
   const int t = threadIdx.x;
   const int64_t g = base + t;
-  if (g < n) {
+  bool wide = false;                                   // uniform over the grid
+  if constexpr (LANES > 1) wide = row_ptr[nC * P] - row_ptr[0] >= kAffLong * nC * P;
+  if constexpr (LANES > 1) {
+    if (wide) {
+      const int64_t r = base + t / LANES;
+      const int64_t b = r < n ? r / ((int64_t)nC * P) : 0;
+      const int row = r < n ? (int)(r - b * nC * P) : 0;
+      const int k0 = row_ptr[row], k1 = r < n ? row_ptr[row + 1] : k0;
+      const float acc = wide_row_sum<ROWS, LANES>(k0, k1, theta + b * d, col_idx, vals);
+      if (t % LANES == 0) {
+        if (r < n) As[r] = acc;
+        tile[t / LANES] = acc;
+      }
+    }
+  }
+  if (!wide && t < ROWS && g < n) {
     const int64_t b = g / ((int64_t)nC * P);
     const int row = (int)(g - b * nC * P);
     const float* th = theta + b * d;
@@ -507,7 +587,7 @@ __global__ __launch_bounds__(kAffCells<D> * D * (D + 1)) void affine_expm_kernel
     for (int k = 0; k < P; ++k) tile[t * P + k] = r[k];  // only this thread uses these slots
   }
   __syncthreads();
-  if (g < n) Trels[g] = tile[t];
+  if (t < ROWS && g < n) Trels[g] = tile[t];
 }
 
 inline unsigned grid_for(int64_t n, int block) {
@@ -550,14 +630,22 @@ hipError_t launch_affine_expm(int ndim, int64_t n_theta, int nC, int d, const fl
                               float dT, float* As, float* Trels, hipStream_t s) {
   const int64_t n = n_theta * nC;
   if (n <= 0) return hipSuccess;
-  auto go = [&](auto kernel, int cells, int P) {
-    const dim3 g((unsigned)((n + cells - 1) / cells)), b((unsigned)(cells * P));
+  auto go = [&](auto kernel, int cells, int threads) {
+    const dim3 g((unsigned)((n + cells - 1) / cells)), b((unsigned)threads);
     hipLaunchKernelGGL(kernel, g, b, 0, s, n_theta, nC, d, theta, row_ptr, col_idx, vals, dT, As,
                        Trels);
   };
-  if (ndim == 1) go(affine_expm_kernel<1>, kAffCells<1>, 2);
-  else if (ndim == 2) go(affine_expm_kernel<2>, kAffCells<2>, 6);
-  else go(affine_expm_kernel<3>, kAffCells<3>, 12);
+#define CPAB_AFFINE(D, L) go(affine_expm_kernel<D, L>, kAffCells<D, L>, kAffThreads<D, L>)
+  if (n <= kAffFew) {
+    if (ndim == 1) CPAB_AFFINE(1, kAffLanes);
+    else if (ndim == 2) CPAB_AFFINE(2, kAffLanes);
+    else CPAB_AFFINE(3, kAffLanes);
+  } else {
+    if (ndim == 1) CPAB_AFFINE(1, 1);
+    else if (ndim == 2) CPAB_AFFINE(2, 1);
+    else CPAB_AFFINE(3, 1);
+  }
+#undef CPAB_AFFINE
   return hipGetLastError();
 }
 

@@ -1,0 +1,35 @@
+"""The fused affine + exponential launch for few and many matrices and for rows of
+few and many entries: equal to the oracle's sums and to the separate launches
+bit for bit, at counts that do not fill a workgroup and on both sides of the
+4096 matrices where the shape changes."""
+import numpy as np
+import pytest
+import torch
+
+from cpab import Cpab
+from cpab.pytorch._native import native
+from cpab.pytorch.transformer import basis_tables
+from oracle import oracle as orc
+
+from helpers import seeded_theta
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("tess,n,free", [([3, 3], 1, True), ([5, 3], 3, True), ([8, 8], 16, True),
+                                         ([8, 8], 17, True), ([8, 8], 16, False), ([1, 1], 1, False),
+                                         ([2, 1, 3], 1, True), ([3, 3, 3], 5, True),
+                                         ([4, 3, 2], 35, False), ([7], 3, True)])
+def test_affine_expm_shapes(cuda, tess, n, free):
+    T = Cpab(tess, zero_boundary=not free)
+    nd = len(tess)
+    theta = torch.from_numpy(seeded_theta(T, n, 0.3, 950 + n)).to(cuda)
+    tab = basis_tables(T.params, cuda)
+    As = torch.full((n, T.params.nC, nd, nd + 1), float("nan"), device=cuda)
+    Tr, ref_Tr = torch.full_like(As, float("nan")), torch.empty_like(As)
+    native().affine_expm(nd, theta, T.params.nC, tab["row_ptr"], tab["col_idx"], tab["vals"],
+                         1.0 / 50, As, Tr)
+    ref = orc.affine(theta.cpu().numpy(), T.params.basis).reshape(As.shape)
+    np.testing.assert_array_equal(As.cpu().numpy(), ref)
+    native().expm(nd, As, 1.0 / 50, ref_Tr)
+    assert torch.equal(Tr, ref_Tr)
