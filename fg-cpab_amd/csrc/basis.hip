@@ -13,6 +13,7 @@
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <algorithm>
+#include <type_traits>
 #include "cpab_device.hpp"
 #include "cpab_launch.hpp"
 
@@ -43,16 +44,23 @@ __global__ void affine_kernel(int64_t n_theta, int rows, int d, const float* __r
 }
 
 // acc + e[0].x * e[0].y + ... + e[n - 1].x * e[n - 1].y from LDS, one fma after
-// the other.
+// the other.  Bound by that chain and the wait for LDS before each group: groups
+// of 16, where groups of 4 took 30 % longer over columns of 1620 entries and 16
+// more pairs kept in registers ahead cost more moves than they saved.
 __device__ __forceinline__ float add_in_order(const float2* e, int n, float acc) {
   int k = 0;
-  for (; k + 4 <= n; k += 4) {
-    const float2 e0 = e[k], e1 = e[k + 1], e2 = e[k + 2], e3 = e[k + 3];
-    acc = fmaf(e0.x, e0.y, acc);
-    acc = fmaf(e1.x, e1.y, acc);
-    acc = fmaf(e2.x, e2.y, acc);
-    acc = fmaf(e3.x, e3.y, acc);
-  }
+  const auto some = [&](auto count) {
+    constexpr int U = decltype(count)::value;
+    for (; k + U <= n; k += U) {
+      float2 x[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) x[u] = e[k + u];
+#pragma unroll
+      for (int u = 0; u < U; ++u) acc = fmaf(x[u].x, x[u].y, acc);
+    }
+  };
+  some(std::integral_constant<int, 16>{});
+  some(std::integral_constant<int, 4>{});
   for (; k < n; ++k) acc = fmaf(e[k].x, e[k].y, acc);
   return acc;
 }
@@ -64,7 +72,11 @@ __device__ __forceinline__ float add_in_order(const float2* e, int n, float acc)
 // entry by entry from one lane made the projection a chain of dependent
 // memory round trips), stage the (value, moment) pairs in LDS, and the
 // segment's first lane adds them in order.  Columns longer than kProjCap
-// entries take several rounds.
+// entries (a field free at the boundary has up to 382 at [8, 8]) take several
+// rounds, each one's entries loaded during the round before.  8 thetas at
+// [8, 8], free: 12.2 us with groups of 4 and every round's loads at its start,
+// 8.9 so; 4 at [3, 3, 3], free: 46.7 and 31.8; columns of 13 to 54 entries 4.0
+// either way.
 constexpr int kProjSeg = 16;                        // lanes per column
 constexpr int kProjThreads = 256;
 constexpr int kProjCols = kProjThreads / kProjSeg;  // columns per workgroup
@@ -74,7 +86,7 @@ __global__ __launch_bounds__(kProjThreads) void project_kernel(
     int64_t n_theta, int D, int d, const float* __restrict__ M, const int32_t* __restrict__ col_ptr,
     const int32_t* __restrict__ row_idx, const float* __restrict__ vals, float* __restrict__ grad) {
   constexpr int PER = kProjCap / kProjSeg;  // entries per lane per round
-  __shared__ float2 stage[kProjCols][kProjCap];
+  __shared__ float2 stage[kProjCols][kProjCap + 1];   // a wave's columns start two banks apart
   const int seg = threadIdx.x / kProjSeg, lane = threadIdx.x % kProjSeg;
   const int64_t i = blockIdx.x * (int64_t)kProjCols + seg;
   const bool live = i < n_theta * d;
@@ -90,30 +102,33 @@ __global__ __launch_bounds__(kProjThreads) void project_kernel(
   if (lane == 0 && rounds > 0) atomicMax(&max_rounds, rounds);
   __syncthreads();
   rounds = max_rounds;
+  // Every load is issued from an in-range index (entries past the column end
+  // re-read its last entry, which is not added), so a lane's loads are
+  // independent of each other; the next round's are issued before this round's
+  // sum.
+  int idx[PER];
+  float v[PER], mv[PER];
+  const auto load = [&](int from) {
+    if (from >= k1) return;
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+      const int k = min(from + lane + u * kProjSeg, k1 - 1);
+      idx[u] = row_idx[k];
+      v[u] = vals[k];
+    }
+  };
+  load(k0);
   float acc = 0.0f;
   for (int r = 0; r < rounds; ++r) {
     const int base = k0 + r * kProjCap;
     if (base < k1) {
-      // Every load is issued from an in-range index (entries past the column
-      // end re-read its last entry) and masked afterwards, so a lane's loads
-      // are independent of each other.
-      int idx[PER];
-      float v[PER], mv[PER];
-#pragma unroll
-      for (int u = 0; u < PER; ++u) {
-        const int k = min(base + lane + u * kProjSeg, k1 - 1);
-        idx[u] = row_idx[k];
-        v[u] = vals[k];
-      }
 #pragma unroll
       for (int u = 0; u < PER; ++u) mv[u] = m[idx[u]];
 #pragma unroll
-      for (int u = 0; u < PER; ++u) {
-        const bool ok = base + lane + u * kProjSeg < k1;
-        stage[seg][lane + u * kProjSeg] = make_float2(ok ? v[u] : 0.0f, ok ? mv[u] : 0.0f);
-      }
+      for (int u = 0; u < PER; ++u) stage[seg][lane + u * kProjSeg] = make_float2(v[u], mv[u]);
     }
     __syncthreads();
+    load(base + kProjCap);
     if (lane == 0 && base < k1) acc = add_in_order(stage[seg], min(kProjCap, k1 - base), acc);
     __syncthreads();
   }

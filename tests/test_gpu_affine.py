@@ -1,7 +1,8 @@
 """The fused affine + exponential launch for few and many matrices and for rows of
 few and many entries: equal to the oracle's sums and to the separate launches
 bit for bit, at counts that do not fill a workgroup and on both sides of the
-4096 matrices where the shape changes."""
+4096 matrices where the shape changes.  And the projection over columns of several
+rounds (128 entries each)."""
 import numpy as np
 import pytest
 import torch
@@ -33,3 +34,15 @@ def test_affine_expm_shapes(cuda, tess, n, free):
     np.testing.assert_array_equal(As.cpu().numpy(), ref)
     native().expm(nd, As, 1.0 / 50, ref_Tr)
     assert torch.equal(Tr, ref_Tr)
+
+
+@pytest.mark.parametrize("tess,n", [([3, 3], 1), ([8, 8], 3), ([6, 7], 2), ([3, 3, 3], 2), ([2, 1, 3], 5)])
+def test_project_long_columns(cuda, tess, n):
+    T = Cpab(tess, zero_boundary=False)
+    p = T.params
+    tab = basis_tables(p, cuda)
+    M = np.random.default_rng(960).standard_normal((n, p.D)).astype(np.float32)
+    out = torch.full((n, p.d), float("nan"), device=cuda)
+    native().project(torch.from_numpy(M).to(cuda), p.D, p.d, tab["col_ptr"], tab["row_idx"],
+                     tab["vals_t"], out)
+    np.testing.assert_array_equal(out.cpu().numpy(), orc.project(M, p.basis))
