@@ -27,6 +27,7 @@ as the saved final points.
 import torch
 
 from ._native import torch_binding
+from ._tracing import recorded
 
 __all__ = ["CPAB_transformer", "CPAB_chain_transformer", "CPAB_transform_data"]
 
@@ -45,6 +46,10 @@ def CPAB_transformer(points, theta, params, compute_points_grad=False):
     assert points.is_cuda and theta.is_cuda, "Only GPU tensors supported"
     assert params.ndim in (1, 2, 3), "GPU transformer supports 1D, 2D, and 3D"
     assert type(compute_points_grad) == bool, "compute_points_grad must be bool"
+    return recorded(_grid, points, theta, params, compute_points_grad)
+
+
+def _grid(points, theta, params, compute_points_grad):
     return torch_binding().grid(points, theta, params, basis_tables(params, theta.device),
                                 compute_points_grad)
 
@@ -97,6 +102,10 @@ def CPAB_chain_transformer(points, theta_stages, params):
     """
     assert points.is_cuda and theta_stages.is_cuda, "Only GPU tensors supported"
     assert params.ndim in (1, 2, 3), "GPU transformer supports 1D, 2D, and 3D"
+    return recorded(_chain, points, theta_stages, params)
+
+
+def _chain(points, theta_stages, params):
     return torch_binding().chain(points, theta_stages, params,
                                  basis_tables(params, theta_stages.device))
 
@@ -118,7 +127,11 @@ def CPAB_transform_data(data, theta, axes, outsize, params):
     """
     assert data.is_cuda and theta.is_cuda and axes.is_cuda, "Only GPU tensors supported"
     assert params.ndim in (1, 2, 3), "GPU transformer supports 1D, 2D, and 3D"
-    return _CPABImageFunction.forward(None, data, theta, axes, [int(v) for v in outsize], params)
+    return recorded(_image, data, theta, axes, [int(v) for v in outsize], params)
+
+
+def _image(data, theta, axes, outsize, params):
+    return _CPABImageFunction.forward(None, data, theta, axes, outsize, params)
 
 
 class _CPABImageFunction:

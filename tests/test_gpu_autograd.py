@@ -1,7 +1,7 @@
 """The native autograd functions as autograd sees them: second derivatives refused,
 saved-tensor hooks, in-place changes of a saved input, functional transforms and
 forward mode refused, the deterministic setting read when the backward runs,
-side streams, and a used Cpab object copied and pickled."""
+side streams, traced modules, and a used Cpab object copied and pickled."""
 import copy
 import pickle
 
@@ -100,3 +100,23 @@ def test_side_stream(cuda):
     s.synchronize()
     assert torch.equal(out, ref_out)
     torch.testing.assert_close(g, ref, rtol=1e-4, atol=1e-5 * ref.abs().max().item())
+
+
+def test_jit_trace(cuda, tmp_path):
+    # a traced module computes with the inputs it is given, and differentiates
+    T = Cpab([3, 4])
+    for name, f, x in _calls(T, cuda):
+        x.requires_grad_(False)   # a trace keeps it as a constant
+        th, other = _theta(T, cuda), (0.5 * _theta(T, cuda)).detach().requires_grad_()
+        f(th)                     # the first call makes tables that a trace's check would miss
+        m = torch.jit.trace(lambda t: f(2 * t).sin(), (th,))
+        out, ref = m(other), f(2 * other).sin()
+        assert torch.equal(out, ref), name
+        for _ in range(2):
+            got = torch.autograd.grad(out.sum(), other, retain_graph=True)[0]
+            want = torch.autograd.grad(ref.sum(), other, retain_graph=True)[0]
+            torch.testing.assert_close(got, want, rtol=2e-5, atol=1e-6 * want.abs().max().item())
+        with torch.no_grad():
+            assert torch.equal(torch.jit.trace(f, (th,))(other), f(other)), name
+        with pytest.raises(RuntimeError, match="export"):
+            torch.jit.save(m, str(tmp_path / "m.pt"))
