@@ -322,8 +322,12 @@ __device__ __forceinline__ void expm_cell2(const float* A, float dT, float* out)
   out[1] = m01 * exprel;
 }
 
+// A norm that overflows gets as many squarings as the largest finite one (the
+// root of a sum of squares, below 2^64), not the integer its infinity converts
+// to: 2^31 - 1 rounds would hold the device for minutes.
+constexpr float kMostSquarings = 65.0f;
 __device__ __forceinline__ int n_squarings(float norm) {
-  return (norm > 0.5f) ? (int)ceilf(log2f(norm * 2.0f)) : 0;
+  return (norm > 0.5f) ? (int)fminf(ceilf(log2f(norm * 2.0f)), kMostSquarings) : 0;
 }
 
 // Pade(3,3) with scaling and squaring: R = Q^{-1} P, P/Q = I +- M/2 + M^2/12.

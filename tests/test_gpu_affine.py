@@ -1,8 +1,8 @@
 """The fused affine + exponential launch for few and many matrices and for rows of
 few and many entries: equal to the oracle's sums and to the separate launches
 bit for bit, at counts that do not fill a workgroup and on both sides of the
-4096 matrices where the shape changes.  And the projection over columns of several
-rounds (128 entries each)."""
+4096 matrices where the shape changes.  Exponentials of matrices whose norm
+overflows.  And the projection over columns of several rounds (128 entries each)."""
 import numpy as np
 import pytest
 import torch
@@ -34,6 +34,29 @@ def test_affine_expm_shapes(cuda, tess, n, free):
     np.testing.assert_array_equal(As.cpu().numpy(), ref)
     native().expm(nd, As, 1.0 / 50, ref_Tr)
     assert torch.equal(Tr, ref_Tr)
+
+
+@pytest.mark.parametrize("nd", [2, 3])
+def test_expm_of_overflowing_norms(cuda, nd):
+    # infinite entries, and finite ones whose squares overflow: the launch ends,
+    # and the matrices beside them are what they are alone
+    A = torch.rand(64, nd, nd + 1, device=cuda) - 0.5
+    ref, out = torch.empty_like(A), torch.empty_like(A)
+    native().expm(nd, A, 1.0, ref)
+    bad = A.clone()
+    for k, v in enumerate([float("inf"), -float("inf"), float("nan"), 3e38, -1e30, 2e19]):
+        bad[8 * k + 3, k % nd, k % (nd + 1)] = v
+    native().expm(nd, bad, 1.0, out)
+    same = (bad == A).all(-1).all(-1)
+    assert same.sum() == 64 - 6 and torch.equal(out[same], ref[same])
+    # the largest norm that does not overflow (1.8e19) takes the 65 squarings
+    # that it always took: the identity's translation by it
+    big = torch.zeros(1, nd, nd + 1, device=cuda)
+    big[0, 0, nd] = 1.8e19
+    native().expm(nd, big, 1.0, out[:1])
+    want = torch.eye(nd, nd + 1, device=cuda)
+    want[0, nd] = 1.8e19
+    torch.testing.assert_close(out[0], want)
 
 
 @pytest.mark.parametrize("tess,n", [([3, 3], 1), ([8, 8], 3), ([6, 7], 2), ([3, 3, 3], 2), ([2, 1, 3], 5)])
