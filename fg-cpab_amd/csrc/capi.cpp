@@ -1088,7 +1088,7 @@ static int check_interp(int ndim, int64_t B, int64_t C, const int64_t* in_size,
   const int64_t lim = (1LL << 40) - 1, c1 = C > 0 ? C : 1;
   if (n > 0 && (B > lim / n || B * n > lim / c1)) return fail(CPAB_ERR_INVALID, "problem too large");
   if (ndim >= 2) {
-    // one workgroup per tile, 1D grid (fewer than 2^31 threads)
+    // one workgroup of the gather kernels per tile, 1D grid (fewer than 2^31 threads)
     const int64_t tiles = div_up(out_size[0], cpab::kInterpTile0) *
                           div_up(out_size[ndim - 1], cpab::kInterpTileLast) * B *
                           (ndim == 3 ? out_size[1] : 1);

@@ -48,23 +48,30 @@ struct Shape {
   int tiles0, tilesl;  // tiles along i0 and i_last
 };
 
-// Tile of this workgroup, XCD-aware.  The hardware hands consecutive
+// Tiles of a launch, padded to the same number for each XCD.
+__host__ __device__ inline int64_t padded_tiles(const Shape& s) {
+  const int64_t total = (int64_t)s.tiles0 * s.tilesl * s.B * s.omid;
+  return (total + kXcds - 1) / kXcds * kXcds;
+}
+
+// Tile of workgroup wg, XCD-aware.  The hardware hands consecutive
 // workgroup ids to the 8 XCDs in turn, and each XCD has its own L2; the
 // remap gives XCD x the x-th eighth of the tile list, so an XCD works through
 // whole images (tiles ordered i0 tile, then i_last tile, then b * omid + i_mid)
 // and the gathers of one image share that XCD's L2.  Returns false for the
 // padding workgroups past the last tile.
-__device__ __forceinline__ bool tile_origin(const Shape& s, int& b, int& im, int& t0, int& tl) {
+__device__ __forceinline__ bool tile_origin(const Shape& s, int64_t wg, int& b, int& im, int& t0,
+                                            int& tl) {
   const int64_t total = (int64_t)s.tiles0 * s.tilesl * s.B * s.omid;
   const int64_t per = (total + kXcds - 1) / kXcds;
-  const int64_t n = (int64_t)(blockIdx.x % kXcds) * per + blockIdx.x / kXcds;
+  const int64_t n = (wg % kXcds) * per + wg / kXcds;
   if (n >= total) return false;
   const int64_t plane = (int64_t)s.tiles0 * s.tilesl;
-  const int z = (int)(n / plane);
-  const int r = (int)(n - (int64_t)z * plane);
+  const int64_t z = n / plane;
+  const int r = (int)(n - z * plane);
   const int ty = r / s.tiles0;
-  b = z / s.omid;
-  im = z - b * s.omid;
+  b = (int)(z / s.omid);
+  im = (int)(z - (int64_t)b * s.omid);
   t0 = (r - ty * s.tiles0) * kT0;
   tl = ty * kTL;
   return true;
@@ -112,7 +119,7 @@ __global__ __launch_bounds__(kThreads) void interp_fwd_kernel(Shape s,
                                                               float* __restrict__ out) {
   __shared__ float crd[ND][kTL][kT0 + 1];
   int b, im, t0, tl;
-  if (!tile_origin(s, b, im, t0, tl)) return;
+  if (!tile_origin(s, blockIdx.x, b, im, t0, tl)) return;
   const int n0 = min(kT0, s.o0 - t0), nl = min(kTL, s.olast - tl);
   load_tile<ND>(s, grid, b, im, t0, tl, n0, nl, crd);
   __syncthreads();
@@ -175,7 +182,7 @@ __global__ __launch_bounds__(kThreads) void interp_bwd_kernel(Shape s,
                                                               float* __restrict__ grad_grid) {
   __shared__ float crd[ND][kTL][kT0 + 1];
   int b, im, t0, tl;
-  if (!tile_origin(s, b, im, t0, tl)) return;
+  if (!tile_origin(s, blockIdx.x, b, im, t0, tl)) return;
   const int n0 = min(kT0, s.o0 - t0), nl = min(kTL, s.olast - tl);
   load_tile<ND>(s, grid, b, im, t0, tl, n0, nl, crd);
   __syncthreads();
@@ -306,14 +313,14 @@ struct BoxSink {
 };
 
 template <int ND, bool IMG>
-__global__ __launch_bounds__(kScatterThreads) void scatter_kernel(
-    Shape s, const float* __restrict__ coords, const float* __restrict__ grad_out,
-    float* __restrict__ grad_data) {
-  extern __shared__ __align__(16) double box[];   // kBoxMax; first the tile's coordinates
+__device__ __forceinline__ void scatter_tile(const Shape& s, int64_t wg,
+                                             const float* __restrict__ coords,
+                                             const float* __restrict__ grad_out,
+                                             float* __restrict__ grad_data, double* box) {
   __shared__ int lo[3], hi[3];
   float(*crd)[kTL][kT0 + 1] = reinterpret_cast<float(*)[kTL][kT0 + 1]>(box);
   int b, im, t0, tl;
-  if (!tile_origin(s, b, im, t0, tl)) return;
+  if (!tile_origin(s, wg, b, im, t0, tl)) return;
   const int n0 = min(kT0, s.o0 - t0), nl = min(kTL, s.olast - tl);
   if (threadIdx.x < 3) {
     lo[threadIdx.x] = INT_MAX;
@@ -427,6 +434,22 @@ __global__ __launch_bounds__(kScatterThreads) void scatter_kernel(
   }
 }
 
+// One workgroup per tile up to kScatterGrid workgroups; a launch of more tiles
+// (thin volumes in a large batch) walks them in strides of the grid, which
+// would otherwise pass HIP's limit of 2^32 lanes.
+constexpr int64_t kScatterGrid = 1 << 22;   // a multiple of kXcds
+
+template <int ND, bool IMG>
+__global__ __launch_bounds__(kScatterThreads) void scatter_kernel(
+    Shape s, const float* __restrict__ coords, const float* __restrict__ grad_out,
+    float* __restrict__ grad_data) {
+  extern __shared__ __align__(16) double box[];   // kBoxMax; first the tile's coordinates
+  for (int64_t wg = blockIdx.x; wg < padded_tiles(s); wg += gridDim.x) {
+    scatter_tile<ND, IMG>(s, wg, coords, grad_out, grad_data, box);
+    __syncthreads();   // the next tile takes the box
+  }
+}
+
 // 1D: point order equals output order, one thread per (b, point).
 __global__ __launch_bounds__(kThreads) void interp1d_fwd_kernel(int B, int C, int W, int64_t nP,
                                                                 const float* __restrict__ data,
@@ -499,10 +522,7 @@ Shape make_shape(int ndim, int64_t B, int64_t C, const int64_t* in_size, const i
 
 int aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
-dim3 tile_grid(const Shape& s) {
-  const int64_t total = (int64_t)s.tiles0 * s.tilesl * s.B * s.omid;
-  return dim3((unsigned)((total + kXcds - 1) / kXcds * kXcds));
-}
+dim3 tile_grid(const Shape& s) { return dim3((unsigned)padded_tiles(s)); }
 
 template <bool IMG>
 hipError_t launch_scatter(const Shape& s, const float* coords, const float* grad_out,
@@ -512,8 +532,8 @@ hipError_t launch_scatter(const Shape& s, const float* coords, const float* grad
   auto kernel = s.ndim == 2 ? scatter_kernel<2, IMG> : scatter_kernel<3, IMG>;
   const hipError_t e = allow_lds(reinterpret_cast<const void*>(kernel), lds, allowed[s.ndim - 2]);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(kernel, tile_grid(s), dim3(kScatterThreads), lds, st, s, coords, grad_out,
-                     grad_data);
+  const dim3 grid((unsigned)std::min(padded_tiles(s), kScatterGrid));
+  hipLaunchKernelGGL(kernel, grid, dim3(kScatterThreads), lds, st, s, coords, grad_out, grad_data);
   return hipGetLastError();
 }
 

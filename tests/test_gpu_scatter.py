@@ -1,7 +1,7 @@
 """The data gradient's LDS box: boxes at and beyond its capacity (10,000 positions),
 data of one row or column, partial tiles in both directions, the data gradient
-without the grid gradient, and the image backward's scatter at odd sizes,
-against the oracle within the bound of the other data-gradient tests."""
+without the grid gradient, and the image backward's scatter at odd sizes
+and over more tiles than one launch holds workgroups, against the oracle within the bound of the other data-gradient tests."""
 import numpy as np
 import pytest
 import torch
@@ -52,3 +52,22 @@ def test_image_scatter_odd_sizes(cuda, tess, size):
     # of the largest sums
     for a, b in zip(got, ref):
         assert (a - b).abs().max().item() <= 2e-5 * b.abs().max().item()
+
+
+@pytest.mark.parametrize("tiles", [(1 << 22) - 3, (1 << 22) + 5, (1 << 23) + 11])
+def test_image_scatter_many_tiles(cuda, tiles):
+    # a thin volume: every output is a tile of its own.  One workgroup each
+    # reaches 2^32 lanes at 2^23 tiles; the launch holds 2^22.
+    T = cpab_for([2, 1, 1])
+    size, ins = [1, tiles, 1], (2, 3000, 2)
+    rng = np.random.default_rng(820)
+    data = rng.random((1, 1, *ins)).astype(np.float32)
+    g = rng.standard_normal((1, 1, *size)).astype(np.float32)
+    theta = _dev(seeded_theta(T, 1, 0.5, 821), cuda)
+    x = _dev(data, cuda).requires_grad_()
+    gd = torch.autograd.grad(T.transform_data(x, theta, size), x, _dev(g, cuda))[0]
+    with torch.no_grad():
+        grid = T.transform_grid(T.uniform_meshgrid(size), theta).cpu().numpy()
+    _, rd = orc.interp_backward(3, data, grid, size, g, dtype=np.float64)
+    mag = scatter_magnitude(data.shape, grid, size, g)
+    assert (np.abs(gd.cpu().numpy() - rd) <= 1e-4 * mag + 1e-12).all()
