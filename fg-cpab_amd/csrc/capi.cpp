@@ -441,15 +441,19 @@ int64_t workspace_size_impl(int ndim, int64_t nP, int64_t n_batch, int K, int nC
     if (!det_cfg(g, nP, n_batch, &det)) return 0;
     return backward_workspace(g, nP, n_batch, K, det, true).total;
   }
-  // Whichever variant runs (register, trail or segmented) fits, spread or not.
-  cpab::LaunchCfg reg, seg;
-  if (!backward_cfg(g, nP, n_batch, cpab::kRegSteps, 0, &reg) || !backward_cfg(g, nP, n_batch, 0, 1, &seg))
-    return 0;
-  const int64_t wide = std::min<int64_t>(std::max<int64_t>(1, 4 * device_info().cus / n_batch),
-                                         div_up(nP, least_lanes(g, 768)));
-  reg.chunks = (int)std::max<int64_t>(reg.chunks, wide);
-  return std::max(backward_workspace(g, nP, n_batch, K, reg).total,
-                  backward_workspace(g, nP, n_batch, K, seg).total);
+  // The largest of the shapes a call of these sizes may take: every body (the
+  // step count and adaptive substeps are not arguments here), spread or not.
+  const struct { int T, adaptive; } bodies[] = {
+      {cpab::kRegSteps, 0}, {cpab::kRegSteps, 1}, {1, 0}, {cpab::kMaxSteps, 0}, {1, 1}};
+  int64_t most = 0;
+  for (const auto& body : bodies) {
+    cpab::LaunchCfg cfg;
+    if (!backward_cfg(g, nP, n_batch, body.T, body.adaptive, &cfg)) return 0;
+    const cpab::LaunchCfg wide = spread_cfg(g, nP, n_batch, cfg);
+    most = std::max({most, backward_workspace(g, nP, n_batch, K, cfg).total,
+                     backward_workspace(g, nP, n_batch, K, wide).total});
+  }
+  return most;
 }
 
 // Moments from the backward's per-cell sums, then (optionally) their projection.

@@ -1,6 +1,6 @@
 """The backward's spread launch shapes: short rows, more rows than compute units, odd
-row lengths and rounds, on NaN-prefilled outputs against the oracle; and a
-workspace with room for the unspread shape only."""
+row lengths and rounds, on NaN-prefilled outputs against the oracle; a workspace
+with room for the unspread shape only; and the size of the workspace asked for."""
 import re
 
 import numpy as np
@@ -49,3 +49,19 @@ def test_unspread_workspace(cuda):
     need = int(re.search(r"need (\d+) bytes", str(e.value)).group(1))
     assert need < native().backward_workspace_size(2, 3000, 2, 64)
     _run(cuda, [4, 4], 2, 3000, 50, ws_bytes=need)
+
+
+@pytest.mark.parametrize("nd,nC,n,nP,per_row", [(2, 1600, 16, 125000, 32), (2, 3600, 16, 262144, 16),
+                                               (2, 1024, 1, 262144, 512), (2, 64, 32, 784, 7),
+                                               (3, 625, 8, 40000, 64), (1, 50, 16, 10000, 20)])
+def test_workspace_holds_the_shapes_that_run(cuda, nd, nC, n, nP, per_row):
+    # per_row: the most workgroups that a body takes for a row on 256 CUs, each
+    # with a table of nC x ppc floats (the segmented body's 512-lane workgroups,
+    # one to four for each CU by their LDS, but no more than cover the row; 7 of
+    # 128 lanes, spread, for 784 points).  Beside them the rows' reverse-sweep
+    # tables and a few words for each cell.
+    ppc = nd * (nd + 1)
+    tables = n * per_row * nC * ppc * 4
+    rest = n * nC * (4 * {1: 4, 2: 12, 3: 24}[nd] + 16) + 65536
+    size = native().backward_workspace_size(nd, nP, n, nC)
+    assert tables <= size <= tables + rest
