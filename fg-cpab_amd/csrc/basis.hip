@@ -47,6 +47,7 @@ __global__ void affine_kernel(int64_t n_theta, int rows, int d, const float* __r
 // the other.  Bound by that chain and the wait for LDS before each group: groups
 // of 16, where groups of 4 took 30 % longer over columns of 1620 entries and 16
 // more pairs kept in registers ahead cost more moves than they saved.
+template <int GROUP = 16>
 __device__ __forceinline__ float add_in_order(const float2* e, int n, float acc) {
   int k = 0;
   const auto some = [&](auto count) {
@@ -59,7 +60,7 @@ __device__ __forceinline__ float add_in_order(const float2* e, int n, float acc)
       for (int u = 0; u < U; ++u) acc = fmaf(x[u].x, x[u].y, acc);
     }
   };
-  some(std::integral_constant<int, 16>{});
+  some(std::integral_constant<int, GROUP>{});
   some(std::integral_constant<int, 4>{});
   for (; k < n; ++k) acc = fmaf(e[k].x, e[k].y, acc);
   return acc;
@@ -73,20 +74,31 @@ __device__ __forceinline__ float add_in_order(const float2* e, int n, float acc)
 // memory round trips), stage the (value, moment) pairs in LDS, and the
 // segment's first lane adds them in order.  Columns longer than kProjCap
 // entries (a field free at the boundary has up to 382 at [8, 8]) take several
-// rounds, each one's entries loaded during the round before.  8 thetas at
-// [8, 8], free: 12.2 us with groups of 4 and every round's loads at its start,
-// 8.9 so; 4 at [3, 3, 3], free: 46.7 and 31.8; columns of 13 to 54 entries 4.0
-// either way.
+// rounds.
+//
+// FEW columns leave the chip mostly idle and a column's latency counts: each
+// round's entries are loaded during the round before and added in groups of 16
+// (8 thetas at [8, 8], free: 12.2 us with groups of 4 and every round's loads at
+// its start, 9.0 so; 4 at [3, 3, 3], free: 44.8 and 30.0).  Beyond kProjFew columns
+// for each CU the work and the lanes in flight count: groups of 8 without loads
+// ahead take 72 registers for 88 (7 waves per SIMD for 5), and no run of
+// kProjSeg entries beyond the column is loaded (64 thetas at [48, 48], columns of
+// 13: 63.7 us in the FEW form with all its loads, 46.8 so; 64 at [10, 10, 10],
+// columns of 54: 27.6 and 19.6; 16 at [30, 30]: 8.1 and 6.0).  The two cross between
+// 6,000 (54 entries) and 10,000 columns (13 entries).
 constexpr int kProjSeg = 16;                        // lanes per column
 constexpr int kProjThreads = 256;
 constexpr int kProjCols = kProjThreads / kProjSeg;  // columns per workgroup
 constexpr int kProjCap = 128;                       // entries staged per round
+constexpr int kProjFew = 32;
 
+template <bool FEW>
 __global__ __launch_bounds__(kProjThreads) void project_kernel(
     int64_t n_theta, int D, int d, const float* __restrict__ M, const int32_t* __restrict__ col_ptr,
     const int32_t* __restrict__ row_idx, const float* __restrict__ vals, float* __restrict__ grad) {
   constexpr int PER = kProjCap / kProjSeg;  // entries per lane per round
-  __shared__ float2 stage[kProjCols][kProjCap + 1];   // a wave's columns start two banks apart
+  // groups of 16: a wave's columns start two banks apart; of 8: pairs in 16-byte reads
+  __shared__ float2 stage[kProjCols][kProjCap + (FEW ? 1 : 0)];
   const int seg = threadIdx.x / kProjSeg, lane = threadIdx.x % kProjSeg;
   const int64_t i = blockIdx.x * (int64_t)kProjCols + seg;
   const bool live = i < n_theta * d;
@@ -102,34 +114,52 @@ __global__ __launch_bounds__(kProjThreads) void project_kernel(
   if (lane == 0 && rounds > 0) atomicMax(&max_rounds, rounds);
   __syncthreads();
   rounds = max_rounds;
-  // Every load is issued from an in-range index (entries past the column end
-  // re-read its last entry, which is not added), so a lane's loads are
-  // independent of each other; the next round's are issued before this round's
-  // sum.
-  int idx[PER];
-  float v[PER], mv[PER];
-  const auto load = [&](int from) {
-    if (from >= k1) return;
+  // A round's loads are issued together, from in-range indices (past the
+  // column's end its last entry, which is not added); parts of it beyond the
+  // column are skipped.
+  struct Entries {
+    int idx[PER];
+    float v[PER];
+  };
+  constexpr int PART = FEW ? PER / 2 : 1;   // runs of kProjSeg entries to a branch
+  const auto load = [&](int from, Entries& e) {
 #pragma unroll
-    for (int u = 0; u < PER; ++u) {
-      const int k = min(from + lane + u * kProjSeg, k1 - 1);
-      idx[u] = row_idx[k];
-      v[u] = vals[k];
+    for (int p = 0; p < PER; p += PART) {
+      if (from + p * kProjSeg >= k1) break;
+#pragma unroll
+      for (int u = p; u < p + PART; ++u) {
+        const int k = min(from + lane + u * kProjSeg, k1 - 1);
+        e.idx[u] = row_idx[k];
+        e.v[u] = vals[k];
+      }
     }
   };
-  load(k0);
+  Entries next;
+  if constexpr (FEW) load(k0, next);
   float acc = 0.0f;
   for (int r = 0; r < rounds; ++r) {
     const int base = k0 + r * kProjCap;
-    if (base < k1) {
+    Entries e;
+    if constexpr (FEW) e = next;
+    else load(base, e);
+    float mv[PER];
 #pragma unroll
-      for (int u = 0; u < PER; ++u) mv[u] = m[idx[u]];
+    for (int p = 0; p < PER; p += PART) {
+      if (base + p * kProjSeg >= k1) break;
 #pragma unroll
-      for (int u = 0; u < PER; ++u) stage[seg][lane + u * kProjSeg] = make_float2(v[u], mv[u]);
+      for (int u = p; u < p + PART; ++u) mv[u] = m[e.idx[u]];
+    }
+#pragma unroll
+    for (int p = 0; p < PER; p += PART) {
+      if (base + p * kProjSeg >= k1) break;
+#pragma unroll
+      for (int u = p; u < p + PART; ++u)
+        stage[seg][lane + u * kProjSeg] = make_float2(e.v[u], mv[u]);
     }
     __syncthreads();
-    load(base + kProjCap);
-    if (lane == 0 && base < k1) acc = add_in_order(stage[seg], min(kProjCap, k1 - base), acc);
+    if constexpr (FEW) load(base + kProjCap, next);
+    if (lane == 0 && base < k1)
+      acc = add_in_order<FEW ? 16 : 8>(stage[seg], min(kProjCap, k1 - base), acc);
     __syncthreads();
   }
   if (live && lane == 0) grad[i] = acc;
@@ -670,11 +700,12 @@ hipError_t launch_affine_expm(int ndim, int64_t n_theta, int nC, int d, const fl
 
 hipError_t launch_project(int64_t n_theta, int D, int d, const float* moments,
                           const int32_t* col_ptr, const int32_t* row_idx, const float* vals,
-                          float* grad_theta, hipStream_t s) {
+                          float* grad_theta, int cus, hipStream_t s) {
   const int64_t n = n_theta * d;
   if (n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(project_kernel, dim3(grid_for(n, kProjCols)), dim3(kProjThreads), 0, s,
-                     n_theta, D, d, moments, col_ptr, row_idx, vals, grad_theta);
+  hipLaunchKernelGGL(n <= (int64_t)kProjFew * cus ? project_kernel<true> : project_kernel<false>,
+                     dim3(grid_for(n, kProjCols)), dim3(kProjThreads), 0, s, n_theta, D, d,
+                     moments, col_ptr, row_idx, vals, grad_theta);
   return hipGetLastError();
 }
 

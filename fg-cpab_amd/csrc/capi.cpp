@@ -465,7 +465,7 @@ int finish_and_project(const char* who, int ndim, int64_t rows, int nC, const cp
                      who);
   if (rc || !pr.grad_theta || pr.d == 0) return rc;
   return check_hip(cpab::launch_project(rows, nC * ndim * (ndim + 1), pr.d, moments, pr.col_ptr,
-                                        pr.row_idx, pr.vals, pr.grad_theta, s),
+                                        pr.row_idx, pr.vals, pr.grad_theta, device_info().cus, s),
                    who);
 }
 
@@ -559,7 +559,7 @@ int backward_impl(const char* who, int ndim, int64_t nP, int64_t n_batch, int ba
                    who);
     if (rc || !pr.grad_theta || pr.d == 0) return rc;
     return check_hip(cpab::launch_project(rows, g.nC * g.ppc(), pr.d, moments, pr.col_ptr,
-                                          pr.row_idx, pr.vals, pr.grad_theta, s),
+                                          pr.row_idx, pr.vals, pr.grad_theta, device_info().cus, s),
                      who);
   }
   hipEvent_t ev = nullptr;
@@ -1001,7 +1001,7 @@ int cpab_transform_data_backward(int ndim, int64_t n_batch, int64_t n_channels,
                    who);
     if (rc || !pr.grad_theta || pr.d == 0) return rc;
     return check_hip(cpab::launch_project(n_batch, g.nC * g.ppc(), pr.d, moments, pr.col_ptr,
-                                          pr.row_idx, pr.vals, pr.grad_theta, s),
+                                          pr.row_idx, pr.vals, pr.grad_theta, device_info().cus, s),
                      who);
   }
   rc = check_hip(cpab::launch_image_backward(g, img, n_batch, nstepsolver, adaptive, axes,
@@ -1025,7 +1025,7 @@ int cpab_project(int64_t n_theta, int D, int d, const float* moments, const int3
   CPAB_REQUIRE(moments); CPAB_REQUIRE(col_ptr); CPAB_REQUIRE(row_idx); CPAB_REQUIRE(vals);
   CPAB_REQUIRE(grad_theta);
   return check_hip(cpab::launch_project(n_theta, D, d, moments, col_ptr, row_idx, vals,
-                                        grad_theta, as_stream(stream)),
+                                        grad_theta, device_info().cus, as_stream(stream)),
                    "cpab_project");
 }
 

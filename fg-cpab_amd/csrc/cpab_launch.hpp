@@ -91,7 +91,7 @@ hipError_t launch_affine_expm(int ndim, int64_t n_theta, int nC, int d, const fl
                               float dT, float* As, float* Trels, hipStream_t s);
 hipError_t launch_project(int64_t n_theta, int D, int d, const float* moments,
                           const int32_t* col_ptr, const int32_t* row_idx, const float* vals,
-                          float* grad_theta, hipStream_t s);
+                          float* grad_theta, int cus, hipStream_t s);
 // G [rows, nC, RevStride]: per cell h A + (h^2/2) A^2 and the inverse one-step
 // map (cpab_device.hpp), h = 1/T; amp [rows, adjoint_table_blocks(nC)]: the
 // largest ||M_c||_2 of the inverse maps over each block of a row's cells;

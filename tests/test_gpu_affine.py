@@ -2,7 +2,8 @@
 few and many entries: equal to the oracle's sums and to the separate launches
 bit for bit, at counts that do not fill a workgroup and on both sides of the
 4096 matrices where the shape changes.  Exponentials of matrices whose norm
-overflows.  And the projection over columns of several rounds (128 entries each)."""
+overflows.  And the projection over columns of several rounds (128 entries each)
+and on both sides of the 32 columns for each of 256 CUs where its form changes."""
 import numpy as np
 import pytest
 import torch
@@ -65,6 +66,20 @@ def test_project_long_columns(cuda, tess, n):
     p = T.params
     tab = basis_tables(p, cuda)
     M = np.random.default_rng(960).standard_normal((n, p.D)).astype(np.float32)
+    out = torch.full((n, p.d), float("nan"), device=cuda)
+    native().project(torch.from_numpy(M).to(cuda), p.D, p.d, tab["col_ptr"], tab["row_idx"],
+                     tab["vals_t"], out)
+    np.testing.assert_array_equal(out.cpu().numpy(), orc.project(M, p.basis))
+
+
+@pytest.mark.parametrize("tess,free,n", [([8, 8], True, 28), ([8, 8], True, 29), ([30, 30], False, 2),
+                                         ([30, 30], False, 3), ([3, 3, 3], True, 43),
+                                         ([8, 8, 8], False, 8), ([50], False, 300)])
+def test_project_few_and_many_columns(cuda, tess, free, n):
+    T = Cpab(tess, zero_boundary=not free)
+    p = T.params
+    tab = basis_tables(p, cuda)
+    M = np.random.default_rng(961).standard_normal((n, p.D)).astype(np.float32)
     out = torch.full((n, p.d), float("nan"), device=cuda)
     native().project(torch.from_numpy(M).to(cuda), p.D, p.d, tab["col_ptr"], tab["row_idx"],
                      tab["vals_t"], out)
