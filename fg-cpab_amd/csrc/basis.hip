@@ -532,11 +532,14 @@ __global__ void expm_kernel(int64_t n, float dT, const float* __restrict__ As,
 // One thread walking a long row (a field free at the boundary has 22 entries on
 // average and up to 42 at [8, 8], 72 at [3, 3, 3]) is a chain of memory round
 // trips, each lane of a wave in a cache line of its own, in few workgroups (32
-// for 2048 matrices).  Free fields, before and after: 8 thetas at [8, 8] 19.5 ->
-// 5.4 us, 16 of them 20.8 -> 5.8, 4 at [3, 3, 3] 33.9 -> 6.0.  The small
-// workgroups' exponentials fill an eighth of a wave, so short rows (1 to 3
-// entries, one thread each here too) pay 0.1 to 0.3 us up to 4096 matrices
-// (3.4 -> 3.7); beyond, several rounds of workgroups cost more (with eight
+// for 2048 matrices).  Free fields, before and after: 8 thetas at [8, 8] 18.8 ->
+// 4.8 us, 16 of them 20.0 -> 5.3, 4 at [3, 3, 3] 33.9 -> 5.9.  Short rows (1 to 3
+// entries) take one thread each here too, in the first of the workgroups and
+// with full waves of exponentials; the others end at once.  What is left of the
+// choice is 0.02 to 0.08 us (6 thetas at [5, 5, 5]: 3.43 us in the one-thread shape,
+// 3.50 so, 3.68 with the small workgroups' eighths of waves; 8 at [8, 8]: 3.01,
+// 3.06, 3.03).
+// Beyond 4096 matrices several rounds of small workgroups cost more (with eight
 // threads on short rows as well, 8192: 4.9 -> 7.0 us; 16,384: 3.7 -> 9.7).
 constexpr int kAffLanes = 8;
 constexpr int kAffFew = 4096;
@@ -547,10 +550,18 @@ constexpr int kAffCells = (D == 1 ? 256 : 384) / (D * (D + 1)) / LANES;
 template <int D, int LANES>
 constexpr int kAffThreads = kAffCells<D, LANES> * D * (D + 1) * LANES;
 
-// The sum of the row's entries k0 .. k1 - 1 times theta, by LANES threads per
-// row (whole workgroup; the result is the first one's): they read the entries
-// in coalesced runs, gather their thetas together and stage both in LDS, and the
-// first adds them in order, as project_kernel does.
+// The sum of the row's entries k0 .. k1 - 1 times theta.
+__device__ __forceinline__ float row_sum(int k0, int k1, const float* __restrict__ th,
+                                         const int32_t* __restrict__ col_idx,
+                                         const float* __restrict__ vals) {
+  float acc = 0.0f;
+  for (int k = k0; k < k1; ++k) acc = fmaf(vals[k], th[col_idx[k]], acc);
+  return acc;
+}
+
+// The same by LANES threads per row (whole workgroup; the result is the first
+// one's): they read the entries in coalesced runs, gather their thetas together
+// and stage both in LDS, and the first adds them in order, as project_kernel does.
 template <int ROWS, int LANES>
 __device__ __forceinline__ float wide_row_sum(int k0, int k1, const float* __restrict__ th,
                                               const int32_t* __restrict__ col_idx,
@@ -595,17 +606,24 @@ __global__ __launch_bounds__((kAffThreads<D, LANES>)) void affine_expm_kernel(
     const int32_t* __restrict__ row_ptr, const int32_t* __restrict__ col_idx,
     const float* __restrict__ vals, float dT, float* __restrict__ As, float* __restrict__ Trels) {
   constexpr int P = D * (D + 1);
-  constexpr int CB = kAffCells<D, LANES>;
-  constexpr int ROWS = CB * P;
-  __shared__ float tile[ROWS];
+  constexpr int ROWS = kAffCells<D, LANES> * P;        // of a workgroup with LANES threads per row
+  constexpr int THREADS = kAffThreads<D, LANES>;
+  __shared__ float tile[THREADS];
   const int64_t n = n_theta * nC * P;                  // rows of A in all
-  const int64_t base = (int64_t)blockIdx.x * ROWS;     // first row of this block
   const int t = threadIdx.x;
-  const int64_t g = base + t;
-  bool wide = false;                                   // uniform over the grid
-  if constexpr (LANES > 1) wide = row_ptr[nC * P] - row_ptr[0] >= kAffLong * nC * P;
+  int rows = THREADS;                                  // of this workgroup
+  int64_t base = (int64_t)blockIdx.x * THREADS;        // the first of them
+  int64_t g = base + t;
   if constexpr (LANES > 1) {
-    if (wide) {
+    // The limits of the row that this thread would take alone are read beside
+    // those of the whole table, which decide whether it does.
+    const int64_t own = min(g, n - 1), own_b = own / ((int64_t)nC * P);
+    const int own_row = (int)(own - own_b * nC * P);
+    const int own_k0 = row_ptr[own_row], own_k1 = row_ptr[own_row + 1];
+    if (row_ptr[nC * P] - row_ptr[0] >= kAffLong * nC * P) {   // uniform over the grid
+      rows = ROWS;
+      base = (int64_t)blockIdx.x * ROWS;
+      g = base + t;
       const int64_t r = base + t / LANES;
       const int64_t b = r < n ? r / ((int64_t)nC * P) : 0;
       const int row = r < n ? (int)(r - b * nC * P) : 0;
@@ -615,19 +633,23 @@ __global__ __launch_bounds__((kAffThreads<D, LANES>)) void affine_expm_kernel(
         if (r < n) As[r] = acc;
         tile[t / LANES] = acc;
       }
+    } else if (base >= n) {
+      return;   // the first workgroups hold all rows
     }
-  }
-  if (!wide && t < ROWS && g < n) {
+    if (rows == THREADS && g < n) {
+      const float acc = row_sum(own_k0, own_k1, theta + own_b * d, col_idx, vals);
+      As[g] = acc;
+      tile[t] = acc;
+    }
+  } else if (g < n) {
     const int64_t b = g / ((int64_t)nC * P);
     const int row = (int)(g - b * nC * P);
-    const float* th = theta + b * d;
-    float acc = 0.0f;
-    for (int k = row_ptr[row]; k < row_ptr[row + 1]; ++k) acc = fmaf(vals[k], th[col_idx[k]], acc);
+    const float acc = row_sum(row_ptr[row], row_ptr[row + 1], theta + b * d, col_idx, vals);
     As[g] = acc;
     tile[t] = acc;
   }
   __syncthreads();
-  if (t < CB && base + (int64_t)t * P < n) {
+  if (t < rows / P && base + (int64_t)t * P < n) {
     float a[P], r[P];
 #pragma unroll
     for (int k = 0; k < P; ++k) a[k] = tile[t * P + k];
@@ -636,7 +658,7 @@ __global__ __launch_bounds__((kAffThreads<D, LANES>)) void affine_expm_kernel(
     for (int k = 0; k < P; ++k) tile[t * P + k] = r[k];  // only this thread uses these slots
   }
   __syncthreads();
-  if (t < ROWS && g < n) Trels[g] = tile[t];
+  if (t < rows && g < n) Trels[g] = tile[t];
 }
 
 inline unsigned grid_for(int64_t n, int block) {
