@@ -172,7 +172,7 @@ hipError_t go(const BackwardJob& j, const LaunchCfg& cfg, hipStream_t s) {
   const Cells g{j.geo.nx, j.geo.ny, j.geo.nz};
   const Recover rec{j.amp, adjoint_table_blocks(j.geo.nC),
                     (float)std::pow((double)kRecoverGrowth,
-                                    1.0 / (double)(is_trail(BODY) ? kSeg : j.T)),
+                                    1.0 / (double)(is_trail(BODY) ? std::min(j.T, kSeg) : j.T)),
                     j.edge};
   const dim3 grid((unsigned)cfg.chunks, (unsigned)j.n_batch), block((unsigned)cfg.block);
   // Doubles serve single transforms of point arrays, and those always (see Bins).

@@ -714,7 +714,7 @@ template <> struct Trail<104> {
 // so a recovered position is at most kSeg steps of rounding away from the
 // replayed one (without that, the theta gradient of a [48, 48] field was three
 // times further from its 64-bit value), and a row need only keep the growth
-// bound over kSeg steps.
+// bound over kSeg steps, or over T if those are fewer.
 // Bound by VALU issue and the latency of cell changes, as register_body.  One
 // midpoint pass and table reads only at cell changes, where the segmented body
 // makes two passes and reads an entry at every step: 16 thetas x 60,001 points,

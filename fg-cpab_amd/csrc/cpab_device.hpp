@@ -26,13 +26,14 @@ constexpr int kMaxSteps = 100;
 // position buffer in 26 VGPRs.
 constexpr int kSeg = 8;
 constexpr int kMaxSeg = (kMaxSteps + kSeg - 1) / kSeg;
-// Step count whose backward keeps the whole trajectory in registers (the
-// library default nstepsolver=50); other step counts use the segmented replay.
+// Step count whose backward is unrolled with the whole trajectory's cells in
+// registers (the library default nstepsolver=50); others take the trail body.
 constexpr int kRegSteps = 50;
-// The register backward recovers positions step by step through each cell's
+// The register and trail backwards recover positions step by step through each cell's
 // inverse one-step map M_c, which multiplies the rounding error of a recovered
-// position by up to ||M_c||_2 per step.  It does so only for rows (thetas)
-// whose bound (max_c ||M_c||_2)^T is at most kRecoverGrowth; other rows replay
+// position by up to ||M_c||_2 per step.  They do so only for rows (thetas)
+// whose bound (max_c ||M_c||_2)^n is at most kRecoverGrowth over the n steps
+// between known positions (T; trail: at most kSeg); other rows replay
 // the trajectory from checkpoints, which reproduces the replayed positions
 // exactly.  Measured on a CPU emulation of the recovery (1D/2D/3D rows): the
 // largest position error is about 4e-6 below a bound of 2 (theta ~ N(0, 0.5^2),
