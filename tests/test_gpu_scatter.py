@@ -1,7 +1,8 @@
 """The data gradient's LDS box: boxes at and beyond its capacity (10,000 positions),
 data of one row or column, partial tiles in both directions, the data gradient
 without the grid gradient, and the image backward's scatter at odd sizes
-and over more tiles than one launch holds workgroups, against the oracle within the bound of the other data-gradient tests."""
+and over more tiles than one launch holds workgroups, and the 1D gradients one by
+one and together, against the oracle within the bound of the other data-gradient tests."""
 import numpy as np
 import pytest
 import torch
@@ -71,3 +72,21 @@ def test_image_scatter_many_tiles(cuda, tiles):
     _, rd = orc.interp_backward(3, data, grid, size, g, dtype=np.float64)
     mag = scatter_magnitude(data.shape, grid, size, g)
     assert (np.abs(gd.cpu().numpy() - rd) <= 1e-4 * mag + 1e-12).all()
+
+
+@pytest.mark.parametrize("W,n", [(1, 5), (2, 257), (700, 1000)])
+@pytest.mark.parametrize("want", ["grid", "data", "both"])
+def test_interp1d_gradients(cuda, W, n, want):
+    rng = np.random.default_rng(830 + W)
+    data = rng.random((3, 2, W)).astype(np.float32)
+    grid = (1.4 * rng.random((3, 1, n)) - 0.2).astype(np.float32)   # some outside
+    gout = rng.standard_normal((3, 2, n)).astype(np.float32)
+    gg = torch.full(grid.shape, float("nan"), device=cuda) if want != "data" else None
+    gd = torch.full(data.shape, float("nan"), device=cuda) if want != "grid" else None
+    native().interp_backward(1, _dev(data, cuda), _dev(grid, cuda), (n,), _dev(gout, cuda), gg, gd)
+    rg, rd = orc.interp_backward(1, data, grid, (n,), gout)
+    if gg is not None:   # two channels' products in order: the same bits
+        np.testing.assert_array_equal(gg.cpu().numpy(), rg)
+    if gd is not None:
+        mag = scatter_magnitude(data.shape, grid, (n,), gout)
+        assert (np.abs(gd.cpu().numpy() - rd) <= 1e-4 * mag + 1e-12).all()
