@@ -365,7 +365,8 @@ struct PlainIO {
 // (coalesced seed reads) and 3D in meshgrid order (lanes along coordinate 0:
 // fewer cells per wave than image order, strided seed reads).  Start points
 // come from the per-axis coordinate vectors either way.  GS: where the seed's
-// corner scatter adds grad_data (the deterministic pass; NoScatter otherwise).
+// corner scatter adds grad_data (the deterministic pass, and 1D; NoScatter
+// otherwise).
 template <int D, typename GS = NoScatter>
 struct ImageIO {
   static constexpr bool kMeshOrder = D == 3;
@@ -376,7 +377,7 @@ struct ImageIO {
                                     // grad_data), or null
   const float* __restrict__ gout;   // [C, nP] image gradient of this theta
   const float* __restrict__ data;   // [C, plane_in]
-  GS gdata;                         // [C, plane_in], off (on() false) without grad_data
+  GS gdata;                         // [C, plane_in], off (on() false) where not added here
   __device__ __forceinline__ void walk_index(int i, int (&ix)[3]) const {
     if (D >= 2 && s.walk_tiles) tile_index<D>(s, i, ix);
     else if (kMeshOrder) mesh_index<D>(s, i, ix);

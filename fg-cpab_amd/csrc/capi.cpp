@@ -962,7 +962,7 @@ int cpab_transform_data_backward(int ndim, int64_t n_batch, int64_t n_channels,
   if (rc) return rc;
   if (grad_data) {
     rc = check_hip(cpab::launch_fill(grad_data, n_batch * n_channels * img.plane_in, 0.0f, s), who);
-    if (rc == CPAB_OK && !det)
+    if (rc == CPAB_OK && !det && ndim > 1)
       rc = check_hip(cpab::launch_image_scatter(ndim, img, n_batch, final_points, grad_out,
                                                 grad_data, s),
                      who);
@@ -1006,7 +1006,8 @@ int cpab_transform_data_backward(int ndim, int64_t n_batch, int64_t n_channels,
   }
   rc = check_hip(cpab::launch_image_backward(g, img, n_batch, nstepsolver, adaptive, axes,
                                              final_points, seed_grad, As, G, amp, edge, data,
-                                             grad_out, moments, partials, dense, nullptr, cfg, s),
+                                             grad_out, moments, partials, dense,
+                                             ndim == 1 ? grad_data : nullptr, cfg, s),
                  who);
   prof_end(timed, ev, "image_backward", s);
   if (rc) return rc;

@@ -174,7 +174,7 @@ hipError_t launch_image_backward(const Geometry& g, const ImageShape& img, int64
                                  unsigned long long* det_gsums = nullptr);
 // grad_data [n_batch, C, *in] (zero before) of the image backward from the
 // final points [n_batch, ndim, prod(out)] (image order) and grad_out.
-// launch_image_backward itself adds to grad_data only in its deterministic
+// launch_image_backward itself adds to grad_data in 1D and in its deterministic
 // pass.
 hipError_t launch_image_scatter(int ndim, const ImageShape& img, int64_t n_batch,
                                 const float* final_points, const float* grad_out,

@@ -253,9 +253,12 @@ __device__ __forceinline__ void blend_grad(const float* c, const Axis& ax, const
 // plane (the deterministic backward brings its own sink with the same add()).
 struct FloatScatter {
   float* __restrict__ p;
+  __device__ __forceinline__ constexpr bool on() const { return true; }
+  __device__ __forceinline__ FloatScatter channel(int64_t off) const { return {p + off}; }
   __device__ __forceinline__ void add(int i, float v) const { add_at(p, i, v); }
 };
-// No scatter (the default image backward, whose grad_data has its own kernel).
+// No scatter (the default image backward in 2D and 3D, whose grad_data has its own
+// kernel, and in 1D without grad_data).
 struct NoScatter {
   __device__ __forceinline__ constexpr bool on() const { return false; }
   __device__ __forceinline__ NoScatter channel(int64_t) const { return {}; }

@@ -37,7 +37,7 @@ def test_scatter_box_limits(cuda, ins, outs):
     assert (err <= 1e-4 * mag + 1e-12).all(), float((err / (mag + 1e-30)).max())
 
 
-@pytest.mark.parametrize("tess,size", [([5, 4], (71, 45)), ([3, 2, 2], (19, 6, 37))])
+@pytest.mark.parametrize("tess,size", [([5, 4], (71, 45)), ([3, 2, 2], (19, 6, 37)), ([7], (1013,))])
 def test_image_scatter_odd_sizes(cuda, tess, size):
     # theta and data gradients of the public call against the two-step
     # composition (transform_grid of the meshgrid, then interpolate)
