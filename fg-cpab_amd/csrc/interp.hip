@@ -26,6 +26,8 @@ namespace {
 constexpr int kT0 = kInterpTile0;      // tile extent along i0 (grid rows are contiguous in i0)
 constexpr int kTL = kInterpTileLast;   // tile extent along i_last (output rows are contiguous in i_last)
 constexpr int kThreads = kInterpThreads;
+constexpr int kLogT0 = 5, kLogTL = 5;
+static_assert(kT0 == 1 << kLogT0 && kTL == 1 << kLogTL, "tile extents");
 static_assert(kThreads % kTL == 0 && kT0 % 4 == 0 && 64 % kTL == 0 && kT0 % (kThreads / kTL) == 0,
               "tile shape");
 constexpr int kRows = kThreads / kTL;   // tile rows (along i0) a workgroup covers per pass
@@ -45,24 +47,25 @@ struct Shape {
   int o0, omid, olast;
   int64_t nP;
   int vec4;      // grid rows are 16-byte aligned along i0 (o0 % 4 == 0)
-  int tiles0, tilesl;  // tiles along i0 and i_last
+  int tiles0, tilesm, tilesl;  // tiles along i0, i_mid and i_last
+  int log0, logm, logl;        // log2 of a tile's extent along each
 };
 
 // Tiles of a launch, padded to the same number for each XCD.
 __host__ __device__ inline int64_t padded_tiles(const Shape& s) {
-  const int64_t total = (int64_t)s.tiles0 * s.tilesl * s.B * s.omid;
+  const int64_t total = (int64_t)s.tiles0 * s.tilesl * s.B * s.tilesm;
   return (total + kXcds - 1) / kXcds * kXcds;
 }
 
 // Tile of workgroup wg, XCD-aware.  The hardware hands consecutive
 // workgroup ids to the 8 XCDs in turn, and each XCD has its own L2; the
 // remap gives XCD x the x-th eighth of the tile list, so an XCD works through
-// whole images (tiles ordered i0 tile, then i_last tile, then b * omid + i_mid)
+// whole images (tiles ordered i0 tile, then i_last tile, then i_mid tile and b)
 // and the gathers of one image share that XCD's L2.  Returns false for the
 // padding workgroups past the last tile.
 __device__ __forceinline__ bool tile_origin(const Shape& s, int64_t wg, int& b, int& im, int& t0,
                                             int& tl) {
-  const int64_t total = (int64_t)s.tiles0 * s.tilesl * s.B * s.omid;
+  const int64_t total = (int64_t)s.tiles0 * s.tilesl * s.B * s.tilesm;
   const int64_t per = (total + kXcds - 1) / kXcds;
   const int64_t n = (wg % kXcds) * per + wg / kXcds;
   if (n >= total) return false;
@@ -70,10 +73,10 @@ __device__ __forceinline__ bool tile_origin(const Shape& s, int64_t wg, int& b, 
   const int64_t z = n / plane;
   const int r = (int)(n - z * plane);
   const int ty = r / s.tiles0;
-  b = (int)(z / s.omid);
-  im = (int)(z - (int64_t)b * s.omid);
-  t0 = (r - ty * s.tiles0) * kT0;
-  tl = ty * kTL;
+  b = (int)(z / s.tilesm);
+  im = (int)(z - (int64_t)b * s.tilesm) << s.logm;
+  t0 = (r - ty * s.tiles0) << s.log0;
+  tl = ty << s.logl;
   return true;
 }
 
@@ -286,7 +289,7 @@ __global__ __launch_bounds__(kThreads) void interp_bwd_kernel(Shape s,
 //
 // Bound by atomics: a float add to HBM costs a request per 64-byte row it
 // touches (20 G/s measured; a coalesced wave adds 320 G floats/s).  So a
-// workgroup takes a kT0 x kTL tile of outputs, adds its corners in an LDS box
+// workgroup takes a tile of 1024 outputs, adds its corners in an LDS box
 // over the data positions the tile reaches and adds the box to HBM row by row,
 // lanes along the data's contiguous axis: one coalesced add per data position
 // instead of 2^ND scattered ones per output.  The box is in double because
@@ -299,10 +302,12 @@ __global__ __launch_bounds__(kThreads) void interp_bwd_kernel(Shape s,
 // outputs: 14 us here (41 with the float box), 48 when the image backward added
 // them.
 // IMG: the coordinates are in output order (last axis fastest, the fused
-// transform_data's final points), else in grid order (coordinate 0 fastest).
+// transform_data's final points; image_tile's tiles), else in grid order
+// (coordinate 0 fastest; kT0 x kTL tiles of a slice, as the gather kernels).
 constexpr int kScatterThreads = 512;
-constexpr int kScatterRows = kScatterThreads / kTL;   // tile rows per pass
-constexpr int kScatterPer = kT0 / kScatterRows;       // outputs per lane
+constexpr int kScatterLog = 10;                       // log2 of a tile's outputs
+constexpr int kScatterPer = (1 << kScatterLog) / kScatterThreads;   // outputs per lane
+static_assert(kT0 * kTL == 1 << kScatterLog, "grid-order tiles");
 constexpr int kBoxMax = 10000;   // doubles: 80 KB, two workgroups per CU
 
 struct BoxSink {
@@ -321,23 +326,22 @@ __device__ __forceinline__ void scatter_tile(const Shape& s, int64_t wg,
   float(*crd)[kTL][kT0 + 1] = reinterpret_cast<float(*)[kTL][kT0 + 1]>(box);
   int b, im, t0, tl;
   if (!tile_origin(s, wg, b, im, t0, tl)) return;
-  const int n0 = min(kT0, s.o0 - t0), nl = min(kTL, s.olast - tl);
+  const int n0 = min(1 << s.log0, s.o0 - t0), nm = min(1 << s.logm, s.omid - im);
+  const int nl = min(1 << s.logl, s.olast - tl);
   if (threadIdx.x < 3) {
     lo[threadIdx.x] = INT_MAX;
     hi[threadIdx.x] = -1;
   }
   if constexpr (!IMG) load_tile<ND, kScatterThreads>(s, coords, b, im, t0, tl, n0, nl, crd);
   __syncthreads();
-  const int al = threadIdx.x % kTL;
-  const int w = threadIdx.x / kTL;
   const int64_t plane_in = (int64_t)s.in[0] * s.in[1] * (ND == 3 ? s.in[2] : 1);
   const int64_t plane_out = (int64_t)s.o0 * s.omid * s.olast;
-  const int64_t ostride = (int64_t)s.omid * s.olast;
-  const int64_t o0 = (int64_t)(t0 + w) * ostride + (int64_t)im * s.olast + tl + al;
 
-  // This lane's outputs, and the data positions they reach.
+  // This lane's outputs (consecutive lanes along i_last), and the data positions
+  // they reach.
   Axis at[ND][kScatterPer];
   bool live[kScatterPer];
+  int64_t o[kScatterPer];   // their indices in an output plane
   int mn[ND], mx[ND];
 #pragma unroll
   for (int k = 0; k < ND; ++k) {
@@ -346,13 +350,16 @@ __device__ __forceinline__ void scatter_tile(const Shape& s, int64_t wg,
   }
 #pragma unroll
   for (int j = 0; j < kScatterPer; ++j) {
-    const int a0 = w + j * kScatterRows;
-    live[j] = al < nl && a0 < n0;
+    const int e = threadIdx.x + j * kScatterThreads;
+    const int al = e & ((1 << s.logl) - 1), r = e >> s.logl;
+    const int am = r & ((1 << s.logm) - 1), a0 = r >> s.logm;
+    live[j] = al < nl && am < nm && a0 < n0;
+    o[j] = ((int64_t)(t0 + a0) * s.omid + im + am) * s.olast + tl + al;
 #pragma unroll
     for (int k = 0; k < ND; ++k) {
       float x = 0.0f;
       if (live[j]) {
-        if constexpr (IMG) x = coords[((int64_t)b * ND + k) * s.nP + o0 + j * kScatterRows * ostride];
+        if constexpr (IMG) x = coords[((int64_t)b * ND + k) * s.nP + o[j]];
         else x = crd[k][al][a0];
       }
       at[k][j] = axis_of(x, s.in[k]);
@@ -392,7 +399,7 @@ __device__ __forceinline__ void scatter_tile(const Shape& s, int64_t wg,
         if (!live[j]) continue;
         scatter_to<ND>(s.in, FloatScatter{grad_data + bc * plane_in}, at[0][j], at[1][j],
                        ND == 3 ? at[ND - 1][j] : none,
-                       grad_out[bc * plane_out + o0 + j * kScatterRows * ostride]);
+                       grad_out[bc * plane_out + o[j]]);
       }
     }
     return;
@@ -413,7 +420,7 @@ __device__ __forceinline__ void scatter_tile(const Shape& s, int64_t wg,
     float g[kScatterPer];
 #pragma unroll
     for (int j = 0; j < kScatterPer; ++j)
-      g[j] = live[j] ? grad_out[bc * plane_out + o0 + j * kScatterRows * ostride] : 0.0f;
+      g[j] = live[j] ? grad_out[bc * plane_out + o[j]] : 0.0f;
     __syncthreads();   // the box is clear
 #pragma unroll
     for (int j = 0; j < kScatterPer; ++j)
@@ -511,6 +518,9 @@ Shape make_shape(int ndim, int64_t B, int64_t C, const int64_t* in_size, const i
   s.vec4 = (s.o0 % 4) == 0;
   s.tiles0 = (s.o0 + kT0 - 1) / kT0;
   s.tilesl = (s.olast + kTL - 1) / kTL;
+  s.tilesm = s.omid;
+  s.log0 = kLogT0;
+  s.logl = kLogTL;
   return s;
 }
 
@@ -518,14 +528,42 @@ int aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0
 
 dim3 tile_grid(const Shape& s) { return dim3((unsigned)padded_tiles(s)); }
 
+// Tile of the scatter over an image or volume in output order: 32 x 32, in a
+// volume 8 x 8 x 16, whose box holds 1.8 data positions for each output where
+// 32 x 32 outputs of one slice reach 3.4 (whole pass, one channel, 112^3: 376 us in
+// slices, 365 so, 377 with 8 x 16 x 8; three channels 423, 400, 414), longer along
+// the other axes where the output is thinner (16 volumes of 4 x 300 x 4: 117 us with
+// a workgroup for each slice's 16 outputs, 78 so).
+void image_tile(Shape* s) {
+  const int size[3] = {s->o0, s->omid, s->olast};
+  int want[3] = {5, 0, 5}, most[3];
+  if (s->ndim == 3) { want[0] = 3; want[1] = 3; want[2] = 4; }
+  int bits = 0;
+  for (int k = 0; k < 3; ++k) {
+    most[k] = 0;
+    while (most[k] < kScatterLog && (1 << most[k]) < size[k]) ++most[k];
+    want[k] = std::min(want[k], most[k]);
+    bits += want[k];
+  }
+  for (int k : {2, 0, 1})
+    while (bits < kScatterLog && want[k] < most[k]) { ++want[k]; ++bits; }
+  s->log0 = want[0];
+  s->logm = want[1];
+  s->logl = want[2] + (kScatterLog - bits);   // fewer outputs than a tile's
+  s->tiles0 = ((s->o0 - 1) >> s->log0) + 1;
+  s->tilesm = ((s->omid - 1) >> s->logm) + 1;
+  s->tilesl = ((s->olast - 1) >> s->logl) + 1;
+}
+
 template <bool IMG>
-hipError_t launch_scatter(const Shape& s, const float* coords, const float* grad_out,
-                          float* grad_data, hipStream_t st) {
+hipError_t launch_scatter(Shape s, const float* coords, const float* grad_out, float* grad_data,
+                          hipStream_t st) {
   constexpr size_t lds = kBoxMax * sizeof(double);
   static LdsAllowed allowed[2];
   auto kernel = s.ndim == 2 ? scatter_kernel<2, IMG> : scatter_kernel<3, IMG>;
   const hipError_t e = allow_lds(reinterpret_cast<const void*>(kernel), lds, allowed[s.ndim - 2]);
   if (e != hipSuccess) return e;
+  if (IMG) image_tile(&s);
   const dim3 grid((unsigned)std::min(padded_tiles(s), kScatterGrid));
   hipLaunchKernelGGL(kernel, grid, dim3(kScatterThreads), lds, st, s, coords, grad_out, grad_data);
   return hipGetLastError();

@@ -1,8 +1,8 @@
 """The data gradient's LDS box: boxes at and beyond its capacity (10,000 positions),
 data of one row or column, partial tiles in both directions, the data gradient
-without the grid gradient, and the image backward's scatter at odd sizes
-and over more tiles than one launch holds workgroups, and the 1D gradients one by
-one and together, against the oracle within the bound of the other data-gradient tests."""
+without the grid gradient, the image backward's scatter at odd and thin sizes, more
+tiles than one launch holds workgroups, and the 1D gradients one by one and
+together, against the oracle within the bound of the other data-gradient tests."""
 import numpy as np
 import pytest
 import torch
@@ -55,12 +55,13 @@ def test_image_scatter_odd_sizes(cuda, tess, size):
         assert (a - b).abs().max().item() <= 2e-5 * b.abs().max().item()
 
 
-@pytest.mark.parametrize("tiles", [(1 << 22) - 3, (1 << 22) + 5, (1 << 23) + 11])
-def test_image_scatter_many_tiles(cuda, tiles):
-    # a thin volume: every output is a tile of its own.  One workgroup each
-    # reaches 2^32 lanes at 2^23 tiles; the launch holds 2^22.
+@pytest.mark.parametrize("size", [(1, (1 << 23) + 11, 1), (3, 50001, 2), (2, 3, 40001), (2050, 3, 5),
+                                  (9, 17, 31), (8, 8, 16), (1, 1, 1)])
+def test_image_scatter_thin_volumes(cuda, size):
+    # volumes whose slices hold few outputs (2^23 slices of one: a workgroup of
+    # 512 lanes for each passes the 2^32 lanes of a launch) and partial tiles
     T = cpab_for([2, 1, 1])
-    size, ins = [1, tiles, 1], (2, 3000, 2)
+    size, ins = list(size), (2, 300, 2)
     rng = np.random.default_rng(820)
     data = rng.random((1, 1, *ins)).astype(np.float32)
     g = rng.standard_normal((1, 1, *size)).astype(np.float32)
@@ -69,8 +70,40 @@ def test_image_scatter_many_tiles(cuda, tiles):
     gd = torch.autograd.grad(T.transform_data(x, theta, size), x, _dev(g, cuda))[0]
     with torch.no_grad():
         grid = T.transform_grid(T.uniform_meshgrid(size), theta).cpu().numpy()
-    _, rd = orc.interp_backward(3, data, grid, size, g, dtype=np.float64)
+    _, rd = orc.interp_backward(3, data, grid, size, g)
     mag = scatter_magnitude(data.shape, grid, size, g)
+    assert (np.abs(gd.cpu().numpy() - rd) <= 1e-4 * mag + 1e-12).all()
+
+
+@pytest.mark.parametrize("size", [(1000, 4), (3, 2049), (33, 31), (32, 32), (1, 1)])
+def test_image_scatter_thin_images(cuda, size):
+    T = cpab_for([3, 2])
+    rng = np.random.default_rng(822)
+    data = rng.random((2, 2, 40, 30)).astype(np.float32)
+    g = rng.standard_normal((2, 2, *size)).astype(np.float32)
+    theta = _dev(seeded_theta(T, 2, 0.5, 823), cuda)
+    x = _dev(data, cuda).requires_grad_()
+    gd = torch.autograd.grad(T.transform_data(x, theta, list(size)), x, _dev(g, cuda))[0]
+    with torch.no_grad():
+        grid = T.transform_grid(T.uniform_meshgrid(list(size)), theta).cpu().numpy()
+    _, rd = orc.interp_backward(2, data, grid, list(size), g)
+    mag = scatter_magnitude(data.shape, grid, size, g)
+    assert (np.abs(gd.cpu().numpy() - rd) <= 1e-4 * mag + 1e-12).all()
+
+
+@pytest.mark.parametrize("tiles", [(1 << 22) - 3, (1 << 22) + 5, (1 << 23) - 16])
+def test_scatter_many_tiles(cuda, tiles):
+    # grid order: every slice of one output is a tile; a launch holds 2^22
+    # workgroups, and interpolate takes fewer than 2^23 tiles
+    rng = np.random.default_rng(824)
+    data = rng.random((1, 1, 2, 3000, 2)).astype(np.float32)
+    grid = rng.random((1, 3, tiles)).astype(np.float32)
+    g = rng.standard_normal((1, 1, 1, tiles, 1)).astype(np.float32)
+    gd = torch.full(data.shape, float("nan"), device=cuda)
+    native().interp_backward(3, _dev(data, cuda), _dev(grid, cuda), (1, tiles, 1), _dev(g, cuda),
+                             None, gd)
+    _, rd = orc.interp_backward(3, data, grid, (1, tiles, 1), g)
+    mag = scatter_magnitude(data.shape, grid, (1, tiles, 1), g)
     assert (np.abs(gd.cpu().numpy() - rd) <= 1e-4 * mag + 1e-12).all()
 
 
