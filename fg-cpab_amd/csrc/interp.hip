@@ -81,15 +81,15 @@ __device__ __forceinline__ bool tile_origin(const Shape& s, int64_t wg, int& b, 
 }
 
 // Grid rows of this tile -> LDS crd[k][al][a0] (lanes along i0, float4 when aligned).
-template <int ND, int THREADS = kThreads>
+template <int ND>
 __device__ __forceinline__ void load_tile(const Shape& s, const float* __restrict__ grid, int b,
                                           int im, int t0, int tl, int n0, int nl,
-                                          float (*crd)[kTL][kT0 + 1]) {
+                                          float (*crd)[kTL][kT0 + 1], int threads = kThreads) {
   const int64_t row0 = (int64_t)s.o0 * (im + (int64_t)s.omid * tl) + t0;  // point of (t0, tl)
   const int64_t rstride = (int64_t)s.o0 * s.omid;                        // next i_last
   if (s.vec4 && n0 == kT0) {
     constexpr int Q = kT0 / 4;
-    for (int e = threadIdx.x; e < Q * kTL; e += THREADS) {
+    for (int e = threadIdx.x; e < Q * kTL; e += threads) {
       const int q = e % Q, al = e / Q;
       if (al < nl) {
 #pragma unroll
@@ -104,12 +104,48 @@ __device__ __forceinline__ void load_tile(const Shape& s, const float* __restric
       }
     }
   } else {
-    for (int e = threadIdx.x; e < kT0 * kTL; e += THREADS) {
+    for (int e = threadIdx.x; e < kT0 * kTL; e += threads) {
       const int a0 = e % kT0, al = e / kT0;
       if (a0 < n0 && al < nl) {
 #pragma unroll
         for (int k = 0; k < ND; ++k)
           crd[k][al][a0] = grid[((int64_t)b * ND + k) * s.nP + row0 + al * rstride + a0];
+      }
+    }
+  }
+}
+
+// The tile in crd -> grid rows (lanes along i0, float4 when aligned).
+template <int ND>
+__device__ __forceinline__ void store_tile(const Shape& s, float* __restrict__ grad_grid, int b,
+                                           int im, int t0, int tl, int n0, int nl,
+                                           const float (*crd)[kTL][kT0 + 1],
+                                           int threads = kThreads) {
+  const int64_t row0 = (int64_t)s.o0 * (im + (int64_t)s.omid * tl) + t0;
+  const int64_t rstride = (int64_t)s.o0 * s.omid;
+  if (s.vec4 && n0 == kT0) {
+    constexpr int Q = kT0 / 4;
+    for (int e = threadIdx.x; e < Q * kTL; e += threads) {
+      const int q = e % Q, l = e / Q;
+      if (l < nl) {
+#pragma unroll
+        for (int k = 0; k < ND; ++k) {
+          float4 v;
+          v.x = crd[k][l][4 * q];
+          v.y = crd[k][l][4 * q + 1];
+          v.z = crd[k][l][4 * q + 2];
+          v.w = crd[k][l][4 * q + 3];
+          *reinterpret_cast<float4*>(grad_grid + ((int64_t)b * ND + k) * s.nP + row0 + l * rstride + 4 * q) = v;
+        }
+      }
+    }
+  } else {
+    for (int e = threadIdx.x; e < kT0 * kTL; e += threads) {
+      const int a0 = e % kT0, l = e / kT0;
+      if (a0 < n0 && l < nl) {
+#pragma unroll
+        for (int k = 0; k < ND; ++k)
+          grad_grid[((int64_t)b * ND + k) * s.nP + row0 + l * rstride + a0] = crd[k][l][a0];
       }
     }
   }
@@ -254,34 +290,7 @@ __global__ __launch_bounds__(kThreads) void interp_bwd_kernel(Shape s,
     }
   }
   __syncthreads();
-  const int64_t row0 = (int64_t)s.o0 * (im + (int64_t)s.omid * tl) + t0;
-  const int64_t rstride = (int64_t)s.o0 * s.omid;
-  if (s.vec4 && n0 == kT0) {
-    constexpr int Q = kT0 / 4;
-    for (int e = threadIdx.x; e < Q * kTL; e += kThreads) {
-      const int q = e % Q, l = e / Q;
-      if (l < nl) {
-#pragma unroll
-        for (int k = 0; k < ND; ++k) {
-          float4 v;
-          v.x = crd[k][l][4 * q];
-          v.y = crd[k][l][4 * q + 1];
-          v.z = crd[k][l][4 * q + 2];
-          v.w = crd[k][l][4 * q + 3];
-          *reinterpret_cast<float4*>(grad_grid + ((int64_t)b * ND + k) * s.nP + row0 + l * rstride + 4 * q) = v;
-        }
-      }
-    }
-  } else {
-    for (int e = threadIdx.x; e < kT0 * kTL; e += kThreads) {
-      const int a0 = e % kT0, l = e / kT0;
-      if (a0 < n0 && l < nl) {
-#pragma unroll
-        for (int k = 0; k < ND; ++k)
-          grad_grid[((int64_t)b * ND + k) * s.nP + row0 + l * rstride + a0] = crd[k][l][a0];
-      }
-    }
-  }
+  store_tile<ND>(s, grad_grid, b, im, t0, tl, n0, nl, crd);
 }
 
 // grad_data of 2D / 3D resampling: every output adds its gradient, times each
@@ -304,11 +313,21 @@ __global__ __launch_bounds__(kThreads) void interp_bwd_kernel(Shape s,
 // IMG: the coordinates are in output order (last axis fastest, the fused
 // transform_data's final points; image_tile's tiles), else in grid order
 // (coordinate 0 fastest; kT0 x kTL tiles of a slice, as the gather kernels).
+// GRID: grad_grid too, with interp_bwd_kernel's arithmetic, before the box: one
+// launch and one read of coordinates and gradients where both are wanted (32 x 28
+// x 28 outputs, whole backward: 15.9 us as two kernels, 13.1 so; 16 x 512 x 512
+// 86.0 and 80.5; 128^3 68.8 and 67.4).  At least four waves per SIMD: with the 131
+// registers that 3D takes unbounded one workgroup fits a CU (128^3: 86.8 us).
+// FEW: no tile of the launch has more than kScatterFew outputs (thin or small
+// images): every corner goes to HBM, coordinates and grad_grid past LDS, in
+// workgroups of the tile's size (64 x 8 x 8 outputs 11.4 us with the box, 9.1 so;
+// 16 x 4 x 300 x 4 116 and 41; 100 x 16 x 16 12.2 and 10.2).
 constexpr int kScatterThreads = 512;
 constexpr int kScatterLog = 10;                       // log2 of a tile's outputs
 constexpr int kScatterPer = (1 << kScatterLog) / kScatterThreads;   // outputs per lane
 static_assert(kT0 * kTL == 1 << kScatterLog, "grid-order tiles");
 constexpr int kBoxMax = 10000;   // doubles: 80 KB, two workgroups per CU
+constexpr int kScatterFew = 256;
 
 struct BoxSink {
   double* box;
@@ -317,11 +336,15 @@ struct BoxSink {
   }
 };
 
-template <int ND, bool IMG>
+template <int ND, bool IMG, bool GRID, bool FEW>
 __device__ __forceinline__ void scatter_tile(const Shape& s, int64_t wg,
+                                             const float* __restrict__ data,
                                              const float* __restrict__ coords,
                                              const float* __restrict__ grad_out,
+                                             float* __restrict__ grad_grid,
                                              float* __restrict__ grad_data, double* box) {
+  static_assert(!(IMG && GRID), "grad_grid is in grid order");
+  const int threads = FEW ? (int)blockDim.x : kScatterThreads;
   __shared__ int lo[3], hi[3];
   float(*crd)[kTL][kT0 + 1] = reinterpret_cast<float(*)[kTL][kT0 + 1]>(box);
   int b, im, t0, tl;
@@ -332,8 +355,10 @@ __device__ __forceinline__ void scatter_tile(const Shape& s, int64_t wg,
     lo[threadIdx.x] = INT_MAX;
     hi[threadIdx.x] = -1;
   }
-  if constexpr (!IMG) load_tile<ND, kScatterThreads>(s, coords, b, im, t0, tl, n0, nl, crd);
-  __syncthreads();
+  if constexpr (!FEW) {
+    if constexpr (!IMG) load_tile<ND>(s, coords, b, im, t0, tl, n0, nl, crd, kScatterThreads);
+    __syncthreads();
+  }
   const int64_t plane_in = (int64_t)s.in[0] * s.in[1] * (ND == 3 ? s.in[2] : 1);
   const int64_t plane_out = (int64_t)s.o0 * s.omid * s.olast;
 
@@ -342,6 +367,9 @@ __device__ __forceinline__ void scatter_tile(const Shape& s, int64_t wg,
   Axis at[ND][kScatterPer];
   bool live[kScatterPer];
   int64_t o[kScatterPer];   // their indices in an output plane
+  const auto grid_at = [&](int al, int a0) {   // and in grid order
+    return t0 + a0 + (int64_t)s.o0 * (im + (int64_t)s.omid * (tl + al));
+  };
   int mn[ND], mx[ND];
 #pragma unroll
   for (int k = 0; k < ND; ++k) {
@@ -350,7 +378,7 @@ __device__ __forceinline__ void scatter_tile(const Shape& s, int64_t wg,
   }
 #pragma unroll
   for (int j = 0; j < kScatterPer; ++j) {
-    const int e = threadIdx.x + j * kScatterThreads;
+    const int e = threadIdx.x + j * threads;
     const int al = e & ((1 << s.logl) - 1), r = e >> s.logl;
     const int am = r & ((1 << s.logm) - 1), a0 = r >> s.logm;
     live[j] = al < nl && am < nm && a0 < n0;
@@ -360,6 +388,7 @@ __device__ __forceinline__ void scatter_tile(const Shape& s, int64_t wg,
       float x = 0.0f;
       if (live[j]) {
         if constexpr (IMG) x = coords[((int64_t)b * ND + k) * s.nP + o[j]];
+        else if constexpr (FEW) x = coords[((int64_t)b * ND + k) * s.nP + grid_at(al, a0)];
         else x = crd[k][al][a0];
       }
       at[k][j] = axis_of(x, s.in[k]);
@@ -369,28 +398,64 @@ __device__ __forceinline__ void scatter_tile(const Shape& s, int64_t wg,
       }
     }
   }
-#pragma unroll
-  for (int k = 0; k < ND; ++k) {
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) {
-      mn[k] = min(mn[k], __shfl_xor(mn[k], off));
-      mx[k] = max(mx[k], __shfl_xor(mx[k], off));
-    }
-    if ((threadIdx.x & 63) == 0) {
-      atomicMin(&lo[k], mn[k]);
-      atomicMax(&hi[k], mx[k]);
-    }
-  }
-  __syncthreads();
-  int org[3] = {0, 0, 0}, ext[3] = {1, 1, 1};
-  int64_t area = 1;
-#pragma unroll
-  for (int k = 0; k < ND; ++k) {
-    org[k] = __builtin_amdgcn_readfirstlane(lo[k]);
-    ext[k] = __builtin_amdgcn_readfirstlane(hi[k]) - org[k] + 1;
-    area *= ext[k];
-  }
   const Axis none{0, 0, 0.0f};
+  if constexpr (!FEW) {
+#pragma unroll
+    for (int k = 0; k < ND; ++k) {
+#pragma unroll
+      for (int off = 32; off >= 1; off >>= 1) {
+        mn[k] = min(mn[k], __shfl_xor(mn[k], off));
+        mx[k] = max(mx[k], __shfl_xor(mx[k], off));
+      }
+      if ((threadIdx.x & 63) == 0) {
+        atomicMin(&lo[k], mn[k]);
+        atomicMax(&hi[k], mx[k]);
+      }
+    }
+    __syncthreads();
+  }
+  if constexpr (GRID) {
+    float dd[kScatterPer][3] = {};
+    for (int ch = 0; ch < s.C; ++ch) {
+      const int64_t bc = (int64_t)b * s.C + ch;
+      const ChannelBuf d(data + bc * plane_in, plane_in);
+#pragma unroll
+      for (int j = 0; j < kScatterPer; ++j) {
+        float c[1 << ND];
+        const Axis az = ND == 3 ? at[ND - 1][j] : none;
+        gather<ND>(s.in, d, at[0][j], at[1][j], az, c);
+        const float g = live[j] ? grad_out[bc * plane_out + o[j]] : 0.0f;
+        blend_grad<ND>(c, at[0][j], at[1][j], az, g, dd[j]);
+      }
+    }
+    // The coordinates' slots take their gradients (each lane its own).
+#pragma unroll
+    for (int j = 0; j < kScatterPer; ++j) {
+      if (!live[j]) continue;
+      const int e = threadIdx.x + j * threads, al = e & ((1 << s.logl) - 1), a0 = e >> s.logl;
+#pragma unroll
+      for (int k = 0; k < ND; ++k) {
+        const float v = dd[j][k] * (float)(s.in[k] - 1);
+        if constexpr (FEW) grad_grid[((int64_t)b * ND + k) * s.nP + grid_at(al, a0)] = v;
+        else crd[k][al][a0] = v;
+      }
+    }
+    if constexpr (!FEW) {
+      __syncthreads();
+      store_tile<ND>(s, grad_grid, b, im, t0, tl, n0, nl, crd, kScatterThreads);
+      __syncthreads();   // the box may take their place
+    }
+  }
+  int org[3] = {0, 0, 0}, ext[3] = {1, 1, 1};
+  int64_t area = FEW ? INT64_MAX : 1;
+  if constexpr (!FEW) {
+#pragma unroll
+    for (int k = 0; k < ND; ++k) {
+      org[k] = __builtin_amdgcn_readfirstlane(lo[k]);
+      ext[k] = __builtin_amdgcn_readfirstlane(hi[k]) - org[k] + 1;
+      area *= ext[k];
+    }
+  }
   if (area > kBoxMax) {   // uniform over the workgroup
     for (int ch = 0; ch < s.C; ++ch) {
       const int64_t bc = (int64_t)b * s.C + ch;
@@ -446,13 +511,14 @@ __device__ __forceinline__ void scatter_tile(const Shape& s, int64_t wg,
 // would otherwise pass HIP's limit of 2^32 lanes.
 constexpr int64_t kScatterGrid = 1 << 22;   // a multiple of kXcds
 
-template <int ND, bool IMG>
-__global__ __launch_bounds__(kScatterThreads) void scatter_kernel(
-    Shape s, const float* __restrict__ coords, const float* __restrict__ grad_out,
+template <int ND, bool IMG, bool GRID, bool FEW>
+__global__ __launch_bounds__(kScatterThreads, 4) void scatter_kernel(
+    Shape s, const float* __restrict__ data, const float* __restrict__ coords,
+    const float* __restrict__ grad_out, float* __restrict__ grad_grid,
     float* __restrict__ grad_data) {
   extern __shared__ __align__(16) double box[];   // kBoxMax; first the tile's coordinates
   for (int64_t wg = blockIdx.x; wg < padded_tiles(s); wg += gridDim.x) {
-    scatter_tile<ND, IMG>(s, wg, coords, grad_out, grad_data, box);
+    scatter_tile<ND, IMG, GRID, FEW>(s, wg, data, coords, grad_out, grad_grid, grad_data, box);
     __syncthreads();   // the next tile takes the box
   }
 }
@@ -555,17 +621,31 @@ void image_tile(Shape* s) {
   s->tilesl = ((s->olast - 1) >> s->logl) + 1;
 }
 
-template <bool IMG>
-hipError_t launch_scatter(Shape s, const float* coords, const float* grad_out, float* grad_data,
-                          hipStream_t st) {
-  constexpr size_t lds = kBoxMax * sizeof(double);
-  static LdsAllowed allowed[2];
-  auto kernel = s.ndim == 2 ? scatter_kernel<2, IMG> : scatter_kernel<3, IMG>;
-  const hipError_t e = allow_lds(reinterpret_cast<const void*>(kernel), lds, allowed[s.ndim - 2]);
-  if (e != hipSuccess) return e;
-  if (IMG) image_tile(&s);
+template <int ND, bool IMG, bool GRID>
+hipError_t launch_scatter(Shape s, const float* data, const float* coords, const float* grad_out,
+                          float* grad_grid, float* grad_data, hipStream_t st) {
+  if (IMG) {
+    image_tile(&s);
+  } else {   // lanes for the outputs there are
+    while (s.log0 > 0 && (1 << s.log0) >= 2 * s.o0) --s.log0;
+    while (s.logl > 0 && (1 << s.logl) >= 2 * s.olast) --s.logl;
+  }
+  const int most = std::min(s.o0, 1 << s.log0) * std::min(s.omid, 1 << s.logm) *
+                   std::min(s.olast, 1 << s.logl);   // outputs of a tile
+  const int threads = std::min(std::max(1 << (s.log0 + s.logm + s.logl), 64), kScatterThreads);
   const dim3 grid((unsigned)std::min(padded_tiles(s), kScatterGrid));
-  hipLaunchKernelGGL(kernel, grid, dim3(kScatterThreads), lds, st, s, coords, grad_out, grad_data);
+  if (most <= kScatterFew) {
+    hipLaunchKernelGGL((scatter_kernel<ND, IMG, GRID, true>), grid, dim3(threads), 0, st, s, data,
+                       coords, grad_out, grad_grid, grad_data);
+    return hipGetLastError();
+  }
+  constexpr size_t lds = kBoxMax * sizeof(double);
+  static LdsAllowed allowed;
+  auto kernel = scatter_kernel<ND, IMG, GRID, false>;
+  const hipError_t e = allow_lds(reinterpret_cast<const void*>(kernel), lds, allowed);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(kernel, grid, dim3(kScatterThreads), lds, st, s, data, coords, grad_out,
+                     grad_grid, grad_data);
   return hipGetLastError();
 }
 
@@ -611,12 +691,16 @@ hipError_t launch_interp_backward(int ndim, int64_t B, int64_t C, const int64_t*
                             : interp1d_bwd_kernel<false, true>;
     hipLaunchKernelGGL(kernel, dim3((unsigned)g), dim3(kThreads), 0, st, s.B, s.C, s.in[0], s.nP,
                        data, grid, grad_out, grad_grid, grad_data);
-  } else {
-    if (grad_grid)
-      hipLaunchKernelGGL(ndim == 2 ? interp_bwd_kernel<2> : interp_bwd_kernel<3>, tile_grid(s),
-                         dim3(kThreads), 0, st, s, data, grid, grad_out, grad_grid);
-    if (grad_data)
-      return launch_scatter<false>(s, grid, grad_out, grad_data, st);
+  } else if (grad_grid && grad_data) {
+    return ndim == 2 ? launch_scatter<2, false, true>(s, data, grid, grad_out, grad_grid, grad_data, st)
+                     : launch_scatter<3, false, true>(s, data, grid, grad_out, grad_grid, grad_data, st);
+  } else if (grad_data) {
+    return ndim == 2
+               ? launch_scatter<2, false, false>(s, nullptr, grid, grad_out, nullptr, grad_data, st)
+               : launch_scatter<3, false, false>(s, nullptr, grid, grad_out, nullptr, grad_data, st);
+  } else if (grad_grid) {
+    hipLaunchKernelGGL(ndim == 2 ? interp_bwd_kernel<2> : interp_bwd_kernel<3>, tile_grid(s),
+                       dim3(kThreads), 0, st, s, data, grid, grad_out, grad_grid);
   }
   return hipGetLastError();
 }
@@ -636,7 +720,10 @@ hipError_t launch_image_scatter(int ndim, const ImageShape& img, int64_t n_batch
     hipLaunchKernelGGL((interp1d_bwd_kernel<false, true>), dim3((unsigned)g), dim3(kThreads), 0, st,
                        s.B, s.C, s.in[0], s.nP, nullptr, final_points, grad_out, nullptr, grad_data);
   } else {
-    return launch_scatter<true>(s, final_points, grad_out, grad_data, st);
+    return ndim == 2 ? launch_scatter<2, true, false>(s, nullptr, final_points, grad_out, nullptr,
+                                                      grad_data, st)
+                     : launch_scatter<3, true, false>(s, nullptr, final_points, grad_out, nullptr,
+                                                      grad_data, st);
   }
   return hipGetLastError();
 }

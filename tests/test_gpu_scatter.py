@@ -1,8 +1,8 @@
 """The data gradient's LDS box: boxes at and beyond its capacity (10,000 positions),
 data of one row or column, partial tiles in both directions, the data gradient
 without the grid gradient, the image backward's scatter at odd and thin sizes, more
-tiles than one launch holds workgroups, and the 1D gradients one by one and
-together, against the oracle within the bound of the other data-gradient tests."""
+tiles than one launch holds workgroups, both gradients in one launch, and the 1D
+gradients one by one and together, against the oracle within the bound of the other data-gradient tests."""
 import numpy as np
 import pytest
 import torch
@@ -104,6 +104,29 @@ def test_scatter_many_tiles(cuda, tiles):
                              None, gd)
     _, rd = orc.interp_backward(3, data, grid, (1, tiles, 1), g)
     mag = scatter_magnitude(data.shape, grid, (1, tiles, 1), g)
+    assert (np.abs(gd.cpu().numpy() - rd) <= 1e-4 * mag + 1e-12).all()
+
+
+@pytest.mark.parametrize("ins,outs", [((9, 7), (16, 16)), ((9, 7), (17, 16)), ((30, 40), (1, 1)),
+                                      ((30, 40), (3, 300)), ((30, 40), (300, 3)), ((5, 6, 7), (4, 5, 3)),
+                                      ((5, 6, 7), (40, 3, 7)), ((5, 6, 7), (33, 2, 9)), ((1, 1), (36, 64)),
+                                      ((300, 200), (33, 40)), ((20, 21, 40), (8, 3, 40))])
+def test_both_gradients_in_one_launch(cuda, ins, outs):
+    # at most and beyond 256 outputs of a tile, partial tiles, boxes beyond their
+    # capacity; the grid's gradient as the kernel for it alone gives it
+    nd, B, C = len(ins), 3, 2
+    rng = np.random.default_rng(840 + outs[0])
+    data = rng.random((B, C, *ins)).astype(np.float32)
+    grid = (1.2 * rng.random((B, nd, int(np.prod(outs)))) - 0.1).astype(np.float32)
+    gout = rng.standard_normal((B, C, *outs)).astype(np.float32)
+    gd = torch.full(data.shape, float("nan"), device=cuda)
+    gg, alone = (torch.full(grid.shape, float("nan"), device=cuda) for _ in range(2))
+    args = (nd, _dev(data, cuda), _dev(grid, cuda), outs, _dev(gout, cuda))
+    native().interp_backward(*args, gg, gd)
+    native().interp_backward(*args, alone, None)
+    assert torch.equal(gg, alone)
+    _, rd = orc.interp_backward(nd, data, grid, outs, gout)
+    mag = scatter_magnitude(data.shape, grid, outs, gout)
     assert (np.abs(gd.cpu().numpy() - rd) <= 1e-4 * mag + 1e-12).all()
 
 
