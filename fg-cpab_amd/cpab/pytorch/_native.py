@@ -59,6 +59,8 @@ _SIGNATURES = {
                                               _c_int, _c_int, _c_int, _c_vp, _c_vp, _c_vp, _c_vp,
                                               _c_vp, _c_vp, _c_int, _c_vp, _c_vp, _c_vp, _c_vp,
                                               _c_vp, _c_vp, _c_vp, _c_i64, _c_vp]),
+    "cpab_transform_data_backward_data": (_c_int, [_c_int, _c_i64, _c_i64, _c_vp, _c_vp, _c_vp,
+                                                   _c_vp, _c_vp, _c_vp]),
     "cpab_project": (_c_int, [_c_i64, _c_int, _c_int, _c_vp, _c_vp, _c_vp, _c_vp, _c_vp, _c_vp]),
     "cpab_sum_batch": (_c_int, [_c_i64, _c_i64, _c_vp, _c_vp, _c_vp]),
     "cpab_interp_forward": (_c_int, [_c_int, _c_i64, _c_i64, _c_vp, _c_vp, _c_vp, _c_vp, _c_vp,

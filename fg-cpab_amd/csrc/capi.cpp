@@ -651,8 +651,9 @@ const char* cpab_last_error_string(void) { return g_last_error.c_str(); }
 // 300: the backward entry points can also project the moments onto the basis
 // (cpab_backward_project; projection arguments of the chain and
 // transform_data backwards).  200: the fused transform_data entry points take
-// the uniform grid's per-axis coordinates instead of the meshgrid.
-int cpab_abi_version(void) { return 401; }
+// the uniform grid's per-axis coordinates instead of the meshgrid.  402:
+// cpab_transform_data_backward_data.
+int cpab_abi_version(void) { return 402; }
 
 int cpab_affine(int ndim, int64_t n_theta, int nC, int d, const float* theta,
                 const int32_t* row_ptr, const int32_t* col_idx, const float* vals, float* As,
@@ -1013,6 +1014,26 @@ int cpab_transform_data_backward(int ndim, int64_t n_batch, int64_t n_channels,
   if (rc) return rc;
   return finish_and_project(who, ndim, n_batch, g.nC, cfg, nstepsolver, partials, dense, As,
                             moments, pr, s);
+}
+
+int cpab_transform_data_backward_data(int ndim, int64_t n_batch, int64_t n_channels,
+                                      const int64_t* in_size, const int64_t* out_size,
+                                      const float* final_points, const float* grad_out,
+                                      float* grad_data, void* stream) {
+  cpab::ImageShape img;
+  int rc = image_shape(ndim, n_batch, n_channels, in_size, out_size, &img);
+  if (rc) return rc;
+  if (n_batch == 0) return CPAB_OK;
+  CPAB_REQUIRE(final_points); CPAB_REQUIRE(grad_out); CPAB_REQUIRE(grad_data);
+  if (t_deterministic)
+    return fail(CPAB_ERR_INVALID, "the deterministic grad_data needs cpab_transform_data_backward");
+  hipStream_t s = as_stream(stream);
+  const char* who = "cpab_transform_data_backward_data";
+  rc = check_hip(cpab::launch_fill(grad_data, n_batch * n_channels * img.plane_in, 0.0f, s), who);
+  if (rc) return rc;
+  return check_hip(cpab::launch_image_scatter(ndim, img, n_batch, final_points, grad_out, grad_data,
+                                              s),
+                   who);
 }
 
 void cpab_set_deterministic(int on) { t_deterministic = on ? 1 : 0; }

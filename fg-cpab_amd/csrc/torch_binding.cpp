@@ -324,23 +324,32 @@ struct Image : torch::autograd::Function<Image> {
       const Tensor g = grad_of(grads[0]);
       if (ctx->saved_data["need_data"].toBool()) gdata = at::empty_like(d);
       if (ctx->saved_data["need_theta"].toBool()) gtheta = empty({c.n, c.d}, As);
-      const at::DataPtr moments = scratch(c.n * c.nC * c.ppc() * 4);
       const Deterministic det(c.deterministic());
-      int64_t bytes =
-          cpab_transform_data_backward_workspace_size(c.ndim, c.n, c.outsize.data(), c.nC);
-      if (gdata.defined())
-        bytes += cpab_transform_data_backward_data_workspace_size(c.ndim, c.n, d.size(1),
-                                                                  d.sizes().data() + 2);
-      at::DataPtr ws;
-      if (bytes > 0) ws = scratch(bytes);
-      const bool proj = gtheta.defined();
-      check(cpab_transform_data_backward(
-                c.ndim, c.n, d.size(1), d.sizes().data() + 2, c.outsize.data(), c.T, c.nc[0],
-                c.nc[1], c.nc[2], c.adaptive, in(ax), in(fin), in(seed), in(As), in(d), in(g),
-                proj ? c.d : 0, proj ? c.col_ptr.data_ptr<int32_t>() : nullptr,
-                proj ? c.row_idx.data_ptr<int32_t>() : nullptr, proj ? in(c.vals_t) : nullptr,
-                static_cast<float*>(moments.get()), out(gtheta), out(gdata), ws.get(), bytes, s),
-            "cpab_transform_data_backward");
+      // the data's gradient alone needs no trajectories
+      const bool alone = gdata.defined() && !gtheta.defined() && cpab_deterministic() == 0 &&
+                         c.T >= 1 && c.T <= CPAB_MAX_STEPS;   // other counts are refused below
+      if (alone) {
+        check(cpab_transform_data_backward_data(c.ndim, c.n, d.size(1), d.sizes().data() + 2,
+                                                c.outsize.data(), in(fin), in(g), out(gdata), s),
+              "cpab_transform_data_backward_data");
+      } else {
+        const at::DataPtr moments = scratch(c.n * c.nC * c.ppc() * 4);
+        int64_t bytes =
+            cpab_transform_data_backward_workspace_size(c.ndim, c.n, c.outsize.data(), c.nC);
+        if (gdata.defined())
+          bytes += cpab_transform_data_backward_data_workspace_size(c.ndim, c.n, d.size(1),
+                                                                    d.sizes().data() + 2);
+        at::DataPtr ws;
+        if (bytes > 0) ws = scratch(bytes);
+        const bool proj = gtheta.defined();
+        check(cpab_transform_data_backward(
+                  c.ndim, c.n, d.size(1), d.sizes().data() + 2, c.outsize.data(), c.T, c.nc[0],
+                  c.nc[1], c.nc[2], c.adaptive, in(ax), in(fin), in(seed), in(As), in(d), in(g),
+                  proj ? c.d : 0, proj ? c.col_ptr.data_ptr<int32_t>() : nullptr,
+                  proj ? c.row_idx.data_ptr<int32_t>() : nullptr, proj ? in(c.vals_t) : nullptr,
+                  static_cast<float*>(moments.get()), out(gtheta), out(gdata), ws.get(), bytes, s),
+              "cpab_transform_data_backward");
+      }
     }
     return once({gdata, gtheta, Tensor(), Tensor(), Tensor(), Tensor()}, grads[0]);
   }

@@ -47,7 +47,8 @@ const char* cpab_last_error_string(void);
 
 /* ABI version (major*100 + minor).  400: the transform_data entry points take
  * seed_grad.  401: the deterministic mode (cpab_set_deterministic and the
- * workspace sizes and cpab_interp_backward_ws that go with it). */
+ * workspace sizes and cpab_interp_backward_ws that go with it).  402:
+ * cpab_transform_data_backward_data. */
 int cpab_abi_version(void);
 
 /* A = B theta per theta: As[b, r] = sum_k vals[k] * theta[b, col_idx[k]] over
@@ -286,6 +287,17 @@ int cpab_transform_data_backward(int ndim, int64_t n_batch, int64_t n_channels,
                                  const int32_t* row_idx, const float* vals, float* moments,
                                  float* grad_theta, float* grad_data, void* workspace,
                                  int64_t workspace_bytes, void* stream);
+
+/* cpab_transform_data_backward's grad_data [n_batch, C, *in_size] alone
+ * (overwritten; no counterpart in the reference): the final points that the
+ * forward wrote and the image gradient give it, without the trajectories that
+ * the moments need.  In the default mode only (CPAB_ERR_INVALID in the calling
+ * thread's deterministic mode, whose integer sums need
+ * cpab_transform_data_backward and its workspace). */
+int cpab_transform_data_backward_data(int ndim, int64_t n_batch, int64_t n_channels,
+                                      const int64_t* in_size, const int64_t* out_size,
+                                      const float* final_points, const float* grad_out,
+                                      float* grad_data, void* stream);
 
 /* Border-clamped linear/bilinear/trilinear resampling of data
  * [n_batch, C, *in_size] at grid [n_batch, ndim, prod(out_size)] (coordinate 0

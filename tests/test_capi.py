@@ -280,3 +280,26 @@ def _check_deterministic_interp_limits():
         assert rc == 1 and "workspace too small" in _err(lib)
     finally:
         lib.cpab_set_deterministic(0)
+
+
+def test_data_backward_alone_validation():
+    _run_without_gpu("_check_data_backward_alone_validation")
+
+
+def _check_data_backward_alone_validation():
+    lib = _native.load_library()
+    p = ctypes.c_void_p(16)
+    ins, outs = (ctypes.c_int64 * 2)(8, 8), (ctypes.c_int64 * 2)(5, 7)
+    call = lib.cpab_transform_data_backward_data
+    assert call(2, 0, 1, ins, outs, None, None, None, None) == 0
+    for missing in range(3):
+        rc = call(2, 1, 1, ins, outs, *(None if k == missing else p for k in range(3)), None)
+        assert rc == 1 and "must not be NULL" in _err(lib)
+    assert call(4, 1, 1, ins, outs, p, p, p, None) == 1
+    assert call(2, 65536, 1, ins, outs, p, p, p, None) == 1 and "grid limit" in _err(lib)
+    lib.cpab_set_deterministic(1)
+    try:
+        rc = call(2, 1, 1, ins, outs, p, p, p, None)
+        assert rc == 1 and "deterministic" in _err(lib)
+    finally:
+        lib.cpab_set_deterministic(0)

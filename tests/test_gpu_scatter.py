@@ -1,12 +1,14 @@
 """The data gradient's LDS box: boxes at and beyond its capacity (10,000 positions),
 data of one row or column, partial tiles in both directions, the data gradient
 without the grid gradient, the image backward's scatter at odd and thin sizes, more
-tiles than one launch holds workgroups, both gradients in one launch, and the 1D
-gradients one by one and together, against the oracle within the bound of the other data-gradient tests."""
+tiles than one launch holds workgroups, the data gradient without theta's, both
+gradients in one launch, and the 1D gradients one by one and together, against the
+oracle within the bound of the other data-gradient tests."""
 import numpy as np
 import pytest
 import torch
 
+from cpab import Cpab
 from cpab.pytorch._native import native
 from oracle import oracle as orc
 
@@ -105,6 +107,26 @@ def test_scatter_many_tiles(cuda, tiles):
     _, rd = orc.interp_backward(3, data, grid, (1, tiles, 1), g)
     mag = scatter_magnitude(data.shape, grid, (1, tiles, 1), g)
     assert (np.abs(gd.cpu().numpy() - rd) <= 1e-4 * mag + 1e-12).all()
+
+
+@pytest.mark.parametrize("tess,size", [([5, 4], (71, 45)), ([3, 2, 2], (19, 6, 37)), ([7], (1013,))])
+def test_data_gradient_alone(cuda, tess, size):
+    # without theta's gradient no trajectory is replayed: the same data gradient,
+    # also in the deterministic mode, which keeps its own passes
+    rng = np.random.default_rng(812)
+    T = Cpab(tess)
+    theta = _dev(seeded_theta(T, 2, 0.5, 813), cuda)
+    data = _dev(rng.random((2, 3, *size)).astype(np.float32), cuda).requires_grad_()
+    g = _dev(rng.standard_normal((2, 3, *size)).astype(np.float32), cuda)
+    both = torch.autograd.grad(T.transform_data(data, theta.clone().requires_grad_(), list(size)),
+                               data, g)[0]
+    alone = torch.autograd.grad(T.transform_data(data, theta, list(size)), data, g)[0]
+    assert (alone - both).abs().max().item() <= 2e-5 * both.abs().max().item()
+    T.set_solver_params(deterministic_grad=True)
+    runs = [torch.autograd.grad(T.transform_data(data, th, list(size)), data, g)[0]
+            for th in (theta, theta, theta.clone().requires_grad_())]
+    assert torch.equal(runs[0], runs[1]) and torch.equal(runs[0], runs[2])
+    assert (runs[0] - both).abs().max().item() <= 2e-5 * both.abs().max().item()
 
 
 @pytest.mark.parametrize("ins,outs", [((9, 7), (16, 16)), ((9, 7), (17, 16)), ((30, 40), (1, 1)),
