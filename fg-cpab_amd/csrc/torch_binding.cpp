@@ -377,7 +377,8 @@ Tensor image(const Tensor& data, const Tensor& theta, const Tensor& axes,
   c->n = theta.size(0);
   c->nP = nP;
   c->outsize = std::move(outsize);
-  const bool need_data = data.requires_grad(), need_theta = theta.requires_grad();
+  const bool grad = at::GradMode::is_enabled();   // without it nothing is kept for a backward
+  const bool need_data = grad && data.requires_grad(), need_theta = grad && theta.requires_grad();
   py::gil_scoped_release nogil;
   return Image::apply(data, theta, axes, c, need_data, need_theta);
 }

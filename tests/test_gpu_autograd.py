@@ -120,3 +120,21 @@ def test_jit_trace(cuda, tmp_path):
             assert torch.equal(torch.jit.trace(f, (th,))(other), f(other)), name
         with pytest.raises(RuntimeError, match="export"):
             torch.jit.save(m, str(tmp_path / "m.pt"))
+
+
+def test_no_grad_keeps_nothing(cuda):
+    # evaluating under no_grad with tensors that require gradients allocates what
+    # evaluating plain tensors does
+    T = Cpab([4, 4])
+    img = torch.rand(2, 1, 256, 256, device=cuda)
+    th = _theta(T, cuda)
+
+    def peak(x, t):
+        torch.cuda.synchronize()
+        before = torch.cuda.memory_allocated()
+        torch.cuda.reset_peak_memory_stats()
+        with torch.no_grad():
+            T.transform_data(x, t, [256, 256])
+        return torch.cuda.max_memory_allocated() - before
+    T.transform_data(img, th, [256, 256])
+    assert peak(img.clone().requires_grad_(), th) == peak(img.clone(), th.detach())
