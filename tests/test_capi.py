@@ -303,3 +303,18 @@ def _check_data_backward_alone_validation():
         assert rc == 1 and "deterministic" in _err(lib)
     finally:
         lib.cpab_set_deterministic(0)
+
+
+def test_library_builds_without_torch():
+    # the commands that a C caller's build runs, listed by make (nothing is built):
+    # no Python or no torch leaves the library's, and says what is missing
+    csrc = os.path.join(os.path.dirname(_native.__file__), "..", "..", "csrc")
+
+    def steps(*args):
+        return subprocess.run(["make", "-n", "-B", "-C", csrc, *args], check=True, text=True,
+                              capture_output=True).stdout
+    for args in (("PYTHON=/bin/false",), ("lib", "PYTHON=/bin/false"), ("lib",)):
+        out = steps(*args)
+        assert "libcpab_hip.so" in out and "torch_binding" not in out, args
+    assert "finds no torch" in steps("PYTHON=/bin/false")
+    assert "torch_binding.cpp" in steps()
