@@ -49,11 +49,12 @@ constexpr int kInterpThreads = 256;
 struct LaunchCfg {
   int block;        // threads per workgroup
   int chunks;       // workgroups per theta (gridDim.x)
+  int single;       // 2D forward: one point per lane
   int lds_table;    // backward, segmented variant: stage the per-theta affine table in LDS
   int lds_bins;     // backward: accumulate moments in full LDS bins (per-workgroup partials)
   int lds_cache;    // backward: else accumulate in the hashed LDS cell cache
   int trail;        // backward: the trail body for T <= 64 or T <= 104 (0 = another body)
-  int reg_steps;    // backward: compile-time step count of the register variant (0 = segmented)
+  int reg_steps;    // backward: compile-time step count of the register variant (0 = another body)
   int lds_bins64;   // backward, register and trail variants with full bins: bins of doubles
   int lds_rev;      // and (1D/2D) the reverse-sweep table in LDS too
 };

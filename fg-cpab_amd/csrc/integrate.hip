@@ -489,15 +489,14 @@ hipError_t launch_forward(const Geometry& g, int64_t nP, int64_t n_batch, int ba
     if (adaptive)
       return launch2d(fwd2d_kernel<true, 1>, grid, block, s, (int)nP, batched, T, g.nx,
                              g.ny, K, points, Trels, As, out, stage_points);
-    // One point per lane where two would leave SIMDs without a wave (up to four
-    // waves of single points for each of 1024 SIMDs: 32 x 784 points 13.8 ->
-    // 8.6 us), and for chains, which run every stage of a trajectory in one
+    // One point per lane where two would leave SIMDs without a wave (forward_cfg;
+    // 32 x 784 points 13.8 -> 8.6 us), and for chains, which run every stage of a trajectory in one
     // lane: few points (C5: 262,144, 4 waves per SIMD) leave the kernel
     // latency-bound.  One pass over the points, and no barrier between stages
     // (each wave reads the stage tables through L1/L2 at its own pace; staging
     // them in LDS held every workgroup to its slowest wave at each stage: C5
     // forward 123 -> 116 us).
-    if (K > 1 || nP * n_batch <= 262144) {
+    if (K > 1 || cfg.single) {
       const int64_t need1 = (nP + (int64_t)cfg.block - 1) / (int64_t)cfg.block;
       const dim3 grid1((unsigned)need1, (unsigned)n_batch);
       return launch2d(fwd2d_kernel<false, 1>, grid1, block, s, (int)nP, batched, T, g.nx,
