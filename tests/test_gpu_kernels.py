@@ -305,10 +305,9 @@ def test_backward_parity_strong_field(cuda, tess, kind, scale, recovered):
 @pytest.mark.parametrize("tess,kind,nstep", [([50], "line", 20), ([20, 20], "uniform", 37),
                                              ([30, 30], "mesh", 100), ([4, 4, 4], "uniform", 20),
                                              ([10, 10, 10], "mesh", 37)])
-def test_backward_segmented_steps(cuda, tess, kind, nstep):
-    # nstepsolver != 50 runs the segmented replay (a checkpoint every 8 steps,
-    # replayed per segment; 37 and 20 leave a partial last segment; 100 is the
-    # step cap).
+def test_backward_other_step_counts(cuda, tess, kind, nstep):
+    # nstepsolver != 50 runs the trail body (groups of 8 steps; 37 and 20 leave a
+    # partial first group; 100 is the step cap).
     T = cpab_for(tess)
     nd = len(tess)
     theta = seeded_theta(T, 2, 0.5, 90 + nd)

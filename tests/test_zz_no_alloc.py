@@ -65,7 +65,7 @@ def test_noalloc_matches_workspace_backward(cuda):
     # second call, smaller: fewer cells, thetas and points, batched points
     p, pts, As, g = _case(cuda, [4, 4], 2, 300, True, 302)
     _both(cuda, p, pts, As, g, True)
-    # third: 3D, then the segmented variant (nstepsolver != 50)
+    # third: 3D, then the trail body (nstepsolver != 50)
     p, pts, As, g = _case(cuda, [4, 4, 4], 3, 4000, False, 303)
     _both(cuda, p, pts, As, g, False)
     p, pts, As, g = _case(cuda, [20, 20], 2, 3000, False, 304)
