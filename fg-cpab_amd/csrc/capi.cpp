@@ -228,26 +228,33 @@ int64_t least_lanes(const cpab::Geometry& g, int most) {
 // units idle when a row is short (8 rows of 40,000 points: 160 workgroups of
 // 2048 points) and lanes idle in a last round.  Here a row is cut into
 // `chunks` nearly equal ranges, each covered in equal rounds by as many lanes
-// as that takes, with one to four workgroups for each compute unit (one at a
-// time fits, for large tables), whichever is estimated shortest: a round costs
-// a latency and its lanes (about a third and two thirds of a full round,
-// measured on short rows), a workgroup its tables.
-cpab::LaunchCfg spread_cfg(const cpab::Geometry& g, int64_t nP, int64_t n_theta,
+// as that takes, with a sixteenth to four workgroups for each compute unit (one
+// at a time fits, for large tables), whichever is estimated shortest.  In us, from
+// measured passes: a full round of 1024 lanes takes 2 + 0.12 T in 1D, 3 + 0.31 T in
+// 2D and 5 + 0.55 T in 3D, of which a third is its latency; a workgroup 5 for its
+// start and the clearing and writing of a small table, and more for a larger one; the
+// pass over the partial tables, once for a chain's K stages, 0.047 for each of a
+// row's (1 x 30,000 points, [300], T = 50: 40.2 us in 235 workgroups, whose tables
+// take 11 us to add, 30.5 in the 30 unspread ones, 28.6 so).  More steps never give
+// fewer workgroups, which the workspace's size rests on.
+cpab::LaunchCfg spread_cfg(const cpab::Geometry& g, int64_t nP, int64_t n_theta, int T, int K,
                            const cpab::LaunchCfg& base) {
   if (!base.reg_steps && !base.trail) return base;
   const int64_t cus = device_info().cus, n = std::max<int64_t>(n_theta, 1);
   const int64_t most = std::max<int64_t>(1, div_up(nP, least_lanes(g, base.block)));
+  const double full = g.ndim == 1 ? 2.0 + 0.12 * T : g.ndim == 2 ? 3.0 + 0.31 * T : 5.0 + 0.55 * T;
+  const double tables = 5.0 + (double)g.nC * g.ppc() / 2100.0;
   cpab::LaunchCfg best = base;
   double least = 1e300;
-  for (int k = 1; k <= 4; ++k) {
-    const int64_t want = std::min(std::max<int64_t>(1, k * cus / n), most);
+  for (const int sixteenths : {1, 2, 4, 8, 16, 32, 48, 64}) {
+    const int64_t want = std::min(std::max<int64_t>(1, sixteenths * cus / (16 * n)), most);
     const int64_t per = div_up(nP, want), rounds = div_up(per, base.block);
     const int64_t block = div_up(div_up(per, rounds), 64) * 64;
     const int64_t chunks = div_up(nP, block * rounds);
-    const double tables = 0.25 + (double)g.nC * g.ppc() / 40000.0;
     const double cost = (double)div_up(n * chunks, cus) *
-                        (tables + (double)rounds * (0.35 + 0.65 * (double)block / 1024.0));
-    if (cost < least * 0.98) {
+                            (tables + (double)rounds * full * (0.35 + 0.65 * (double)block / 1024.0)) +
+                        (base.lds_bins ? 0.047 * (double)chunks / K : 0.0);
+    if (cost < least) {
       least = cost;
       best.chunks = (int)chunks;
       best.block = (int)block;
@@ -445,14 +452,15 @@ int64_t workspace_size_impl(int ndim, int64_t nP, int64_t n_batch, int K, int nC
     return backward_workspace(g, nP, n_batch, K, det, true).total;
   }
   // The largest of the shapes a call of these sizes may take: every body (the
-  // step count and adaptive substeps are not arguments here), spread or not.
+  // step count and adaptive substeps are not arguments here) at its most steps,
+  // spread or not.
   const struct { int T, adaptive; } bodies[] = {
-      {cpab::kRegSteps, 0}, {cpab::kRegSteps, 1}, {1, 0}, {cpab::kMaxSteps, 0}, {1, 1}};
+      {cpab::kRegSteps, 0}, {cpab::kRegSteps, 1}, {64, 0}, {cpab::kMaxSteps, 0}, {1, 1}};
   int64_t most = 0;
   for (const auto& body : bodies) {
     cpab::LaunchCfg cfg;
     if (!backward_cfg(g, nP, n_batch, body.T, body.adaptive, &cfg)) return 0;
-    const cpab::LaunchCfg wide = spread_cfg(g, nP, n_batch, cfg);
+    const cpab::LaunchCfg wide = spread_cfg(g, nP, n_batch, body.T, K, cfg);
     most = std::max({most, backward_workspace(g, nP, n_batch, K, cfg).total,
                      backward_workspace(g, nP, n_batch, K, wide).total});
   }
@@ -511,7 +519,7 @@ int backward_impl(const char* who, int ndim, int64_t nP, int64_t n_batch, int ba
     return CPAB_ERR_DEVICE;
   BackwardWorkspace w = backward_workspace(g, nP, n_batch, K, cfg, det);
   if (!det) {   // spread, where the caller's workspace has room for its partial tables
-    const cpab::LaunchCfg wide = spread_cfg(g, nP, n_batch, cfg);
+    const cpab::LaunchCfg wide = spread_cfg(g, nP, n_batch, nstepsolver, K, cfg);
     const BackwardWorkspace ww = backward_workspace(g, nP, n_batch, K, wide);
     if (ww.total <= workspace_bytes || ww.total <= w.total) {
       cfg = wide;
@@ -934,7 +942,7 @@ int cpab_transform_data_backward(int ndim, int64_t n_batch, int64_t n_channels,
     return CPAB_ERR_DEVICE;
   BackwardWorkspace w = backward_workspace(g, img.nP, n_batch, 1, cfg, det);
   if (!det) {   // as backward_impl
-    const cpab::LaunchCfg wide = spread_cfg(g, img.nP, n_batch, cfg);
+    const cpab::LaunchCfg wide = spread_cfg(g, img.nP, n_batch, nstepsolver, 1, cfg);
     const BackwardWorkspace ww = backward_workspace(g, img.nP, n_batch, 1, wide);
     if (ww.total <= workspace_bytes || ww.total <= w.total) {
       cfg = wide;

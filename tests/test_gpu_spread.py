@@ -36,7 +36,9 @@ def _run(cuda, tess, n, nP, T, ws_bytes=None):
 
 @pytest.mark.parametrize("tess,n,nP,T", [([4, 4], 32, 784, 50), ([4, 4], 300, 65, 50), ([4, 4], 1, 63, 20),
                                          ([20, 20], 3, 12501, 50), ([20, 20], 200, 130, 50),
-                                         ([5, 5, 5], 8, 5000, 50), ([3, 3, 3], 2, 40001, 70), ([50], 16, 2001, 50)])
+                                         ([5, 5, 5], 8, 5000, 50), ([3, 3, 3], 2, 40001, 70), ([50], 16, 2001, 50),
+                                         ([300], 1, 30000, 50), ([10, 10], 1, 30000, 3), ([10, 10], 2, 5000, 90),
+                                         ([4, 4, 4], 1, 70000, 8)])
 def test_spread_shapes(cuda, tess, n, nP, T):
     _run(cuda, tess, n, nP, T)
 
