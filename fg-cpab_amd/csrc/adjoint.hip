@@ -13,11 +13,11 @@
 //             the loops over the steps rolled in groups of kSeg: the groups'
 //             cells and start positions are written to and read from VGPRs
 //             at a wave-uniform index.
-//   segmented (any T <= 100; adaptive substeps, more cells, rows beyond the
-//             recovery bound) phase 1 keeps a checkpoint every kSeg steps in
-//             a VGPR shift register; phase 2 replays each segment from its
-//             checkpoint into registers and walks it backwards (the
-//             reference's scheme, cpab_ops_2d.cu:236-263).
+//   segmented (any T <= 100; adaptive substeps, more cells, few steps over a
+//             large 2D table, rows beyond the recovery bound) phase 1 keeps a
+//             checkpoint every kSeg steps in a VGPR shift register; phase 2
+//             replays each segment from its checkpoint into registers and walks
+//             it backwards (the reference's scheme, cpab_ops_2d.cu:236-263).
 // All visit the reference's cells; the positions fed to the sums may differ
 // from the replayed ones by a few ulps in the register and trail variants.
 // In all, phase 2 propagates lambda and accumulates the 2x3 (1x2, 3x4) sum
@@ -227,7 +227,12 @@ hipError_t dispatch(const BackwardJob& j, int adaptive, const LaunchCfg& cfg, hi
     CPAB_GO(false, false, LB, kBodyTrail104);                     \
   } while (0)
   if (!adaptive) {
-    if (!cfg.trail && !cfg.reg_steps) CPAB_GO(false, false, kBinsCache, kBodySegmented);
+    if (!cfg.trail && !cfg.reg_steps) {
+      if constexpr (D == 2) {
+        if (cfg.lds_bins) CPAB_GO(false, false, kBinsFull, kBodySegmented);   // few steps
+      }
+      CPAB_GO(false, false, kBinsCache, kBodySegmented);
+    }
     if constexpr (D <= 2) {
       if (cfg.lds_rev && cfg.lds_bins64) CPAB_STEPS(kBinsRev64);
       if (cfg.lds_rev) CPAB_STEPS(kBinsRev);

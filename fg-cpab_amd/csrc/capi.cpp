@@ -181,7 +181,13 @@ bool backward_cfg(const cpab::Geometry& g, int64_t nP, int64_t n_theta, int T, i
   const bool unrolled = packs && T == cpab::kRegSteps &&
                         (g.ndim <= 2 ? c.lds_bins != 0 : !adaptive);
   c.reg_steps = unrolled ? cpab::kRegSteps : 0;
-  c.trail = packs && !adaptive && !unrolled ? (T <= 64 ? 64 : 104) : 0;
+  // Few steps over a 2D table too large for bins of doubles: the trail saves too
+  // little replay for its larger workgroups (kFewSteps).
+  const int64_t budget = dev.lds - 512;   // the kernel's own few words
+  const int most = nP * n_theta <= 128LL * dev.cus ? 2 * cpab::kFewSteps : cpab::kFewSteps;
+  const bool few = T <= most && g.ndim == 2 && c.lds_bins && 2 * table > budget &&
+                   work != Work::kChain;
+  c.trail = packs && !adaptive && !unrolled && !few ? (T <= 64 ? 64 : 104) : 0;
   const bool reg = unrolled || c.trail;
   // Register and trail variants with full bins: bins of doubles when they fit
   // and the work takes them (backward_body.hpp, Bins), and in 1D/2D the
@@ -190,7 +196,6 @@ bool backward_cfg(const cpab::Geometry& g, int64_t nP, int64_t n_theta, int T, i
   // A chain restages each stage's table: measured slower than L2 reads (C5
   // backward 185 -> 190 us).
   const int64_t rev = (int64_t)g.nC * adj_stride(g.ndim) * 4 + 32;
-  const int64_t budget = dev.lds - 512;   // the kernel's own few words
   c.lds_bins64 = (reg && c.lds_bins && work == Work::kPoints && 2 * table <= budget) ? 1 : 0;
   c.lds_rev = (reg && c.lds_bins && work != Work::kChain &&
                (work == Work::kImage || c.lds_bins64) && g.ndim <= 2 &&

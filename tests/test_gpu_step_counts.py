@@ -35,6 +35,14 @@ def test_backward_step_counts_cache_and_strong(cuda, tess, nstep, n, scale):
     _check(tess, nstep, n, scale, cuda)
 
 
+@pytest.mark.parametrize("tess,nstep,n,scale", [([30, 30], 1, 3000, 0.5), ([30, 30], 4, 20000, 0.5),
+                                                ([30, 30], 5, 20000, 0.5), ([41, 41], 8, 3000, 0.5),
+                                                ([41, 41], 9, 3000, 0.5), ([36, 36], 3, 3000, 6.0)])
+def test_backward_few_steps_large_table(cuda, tess, nstep, n, scale):
+    # the segmented body without adaptive substeps, and both sides of its line
+    _check(tess, nstep, n, scale, cuda)
+
+
 @pytest.mark.parametrize("nstep", [5, 20, 37, 70])
 @pytest.mark.parametrize("tess", [[50], [6, 5], [20, 20], [48, 48], [3, 3, 3], [10, 10, 10]])
 def test_adaptive_step_counts(cuda, tess, nstep):
@@ -47,7 +55,7 @@ def test_adaptive_step_counts(cuda, tess, nstep):
 @pytest.mark.parametrize("tess,ins,outs,C,adaptive,scale", [
     ([10], (50,), (1500,), 2, 0, 0.5), ([6, 5], (40, 48), (36, 48), 1, 0, 0.5),
     ([6, 5], (37, 23), (29, 31), 3, 0, 0.5), ([6, 5], (40, 48), (36, 48), 1, 1, 0.5),
-    ([36, 36], (20, 30), (64, 80), 1, 0, 0.5),      # no room for the reverse table
+    ([36, 36], (20, 30), (64, 80), 1, 0, 0.5),      # no room for the reverse table; few steps
     ([48, 48], (20, 30), (64, 80), 2, 0, 0.5),      # the cell cache
     ([3, 3, 3], (10, 12, 9), (11, 9, 13), 2, 0, 0.5), ([10, 10, 10], (10, 12, 9), (16, 8, 32), 1, 0, 0.5),
     ([6, 5], (40, 48), (36, 48), 2, 0, 8.0), ([3, 3, 3], (10, 12, 9), (6, 8, 32), 1, 0, 8.0)])
