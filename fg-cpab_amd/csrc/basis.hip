@@ -248,7 +248,10 @@ __global__ __launch_bounds__(kTableThreads) void adjoint_table_kernel(
 // workgroup covers kFinCells<D> cells of one row (blockIdx.x = row * nblk +
 // block), one thread per (cell, component): S = the HBM sum in `moments` plus
 // partials[row, w, cell] for every part w set in the row's dense-part mask,
-// added in ascending w (a fixed order), the parts' loads issued in batches;
+// added in a fixed order: the parts' loads are issued in batches of 16 in ascending
+// w, a batch is added up in pairs and the batches in double (one after the other in
+// float, many parts' sum took a rounding for each; all of it in double cost 3 us at
+// 16 parts and 20 at 128);
 // then S and the cell's A go through LDS and each thread forms its component
 // of the moments (cpab_device.hpp, moments_from_s), in place.  Consecutive
 // threads read consecutive floats of each partial table.
@@ -281,7 +284,7 @@ __global__ __launch_bounds__(256) void finish_moments_kernel(
                        : (f == 1u ? INFINITY : f == 2u ? -INFINITY : NAN);
     a_lds[t] = As[idx];
   } else if (live) {
-    float s = moments[idx];
+    double s = (double)moments[idx];
     if (nparts > 0) {
       const int64_t R = (int64_t)nC * P;
       const int NW = (nparts + 63) / 64;
@@ -291,21 +294,23 @@ __global__ __launch_bounds__(256) void finish_moments_kernel(
         uint64_t bits = dense_parts[row * NW + q];
         while (bits) {
           float x[U];
-          bool on[U];
 #pragma unroll
           for (int u = 0; u < U; ++u) {
-            on[u] = bits != 0;
-            const int w = on[u] ? q * 64 + __builtin_ctzll(bits) : 0;
+            const bool on = bits != 0;
+            const int w = on ? q * 64 + __builtin_ctzll(bits) : 0;
             bits &= bits - 1;
-            x[u] = on[u] ? src[w * R] : 0.0f;
+            x[u] = on ? src[w * R] : 0.0f;
           }
 #pragma unroll
-          for (int u = 0; u < U; ++u)
-            if (on[u]) s += x[u];
+          for (int half = U / 2; half >= 1; half /= 2) {
+#pragma unroll
+            for (int u = 0; u < half; ++u) x[u] += x[u + half];
+          }
+          s += (double)x[0];
         }
       }
     }
-    s_lds[t] = s;
+    s_lds[t] = (float)s;
     a_lds[t] = As[idx];
   }
   __syncthreads();

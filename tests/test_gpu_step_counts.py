@@ -43,6 +43,28 @@ def test_backward_few_steps_large_table(cuda, tess, nstep, n, scale):
     _check(tess, nstep, n, scale, cuda)
 
 
+def test_backward_rounding_many_tables(cuda):
+    # one row over as many workgroups as there are compute units, each with a table of
+    # its own: their sum takes one rounding, not one for each table
+    _check_rounding([50], 1, 1, 60000, cuda)
+
+
+def _check_rounding(tess, nstep, n_theta, n, cuda):
+    # The oracle replays the same float positions and adds in double.  What is left is
+    # the roundings of the adjoint, one for each step, and those of a workgroup's table,
+    # of the tables' sum and of the moments formed from it.  Each is at most 2^-24 of its
+    # value, 2^-24 / sqrt(3) in the mean of squares, and over this many points they are
+    # independent of each other.
+    T = cpab_for(tess)
+    theta = seeded_theta(T, n_theta, 0.5, 5)
+    pts = uniform_points(len(tess), n, 6)
+    g = np.ones((n_theta, len(tess), n), np.float32)
+    As, mom, _ = _backward_case(T, theta, pts, g, cuda, nstep=nstep)
+    ref, _ = orc.backward(pts, As, g, tess, nstep)
+    err = np.linalg.norm(mom - ref, axis=(1, 2)) / np.linalg.norm(ref, axis=(1, 2))
+    assert (err <= np.sqrt((nstep + 3) / 3.0) * 2.0 ** -24).all(), err * 2.0 ** 24
+
+
 @pytest.mark.parametrize("nstep", [5, 20, 37, 70])
 @pytest.mark.parametrize("tess", [[50], [6, 5], [20, 20], [48, 48], [3, 3, 3], [10, 10, 10]])
 def test_adaptive_step_counts(cuda, tess, nstep):
