@@ -9,17 +9,18 @@
 //             (with adaptive substeps, whose steps are not fixed affine maps,
 //             the positions are kept in VGPRs too).  One midpoint pass per
 //             trajectory.
-//   trail     (any T, no adaptive substeps, up to 65535 cells) the same with
-//             the loops over the steps rolled in groups of kSeg: the groups'
-//             cells and start positions are written to and read from VGPRs
-//             at a wave-uniform index.
+//   trail     (any T, no adaptive substeps, up to 65535 cells) phase 1 keeps
+//             every cell and the position before each group of kSeg steps,
+//             written to and read from VGPRs at a wave-uniform index; phase 2
+//             replays each group over its cells, without looking them up, and
+//             walks it backwards.
 //   segmented (any T <= 100; adaptive substeps, more cells, few steps over a
 //             large 2D table, rows beyond the recovery bound) phase 1 keeps a
 //             checkpoint every kSeg steps in a VGPR shift register; phase 2
 //             replays each segment from its checkpoint into registers and walks
 //             it backwards (the reference's scheme, cpab_ops_2d.cu:236-263).
 // All visit the reference's cells; the positions fed to the sums may differ
-// from the replayed ones by a few ulps in the register and trail variants.
+// from the replayed ones by a few ulps in the register variant.
 // In all, phase 2 propagates lambda and accumulates the 2x3 (1x2, 3x4) sum
 // S = sum lam (x) [p; 1] of the current cell, flushing it whenever the cell
 // changes, as the reference groups its moment flushes.  The reverse step is the
@@ -31,8 +32,8 @@
 // Moment accumulation on MI355X: each workgroup serves ONE theta and one
 // contiguous range of points (spatially coherent for meshgrid inputs).
 //   full bins  the nC x ppc table fits in LDS: the workgroup keeps a private
-//              copy of that theta's sums there (ds_add_f32, no HBM atomics
-//              while integrating).  At the end a workgroup that touched at
+//              copy of that theta's sums there (ds_add_f64 or ds_add_f32, no
+//              HBM atomics while integrating).  At the end a workgroup that touched at
 //              least a quarter of the cells (random points: every workgroup
 //              touches nearly every cell) stores its whole table as its
 //              partial (plain coalesced stores) and sets its bit in the row's
@@ -74,17 +75,17 @@ namespace {
 // on entry), or, from a dense full-bin workgroup, to its partial table with
 // its dense-part bit set; the reverse-sweep table G holds the same rows
 // (RevStride<D>::S floats per cell).
-// Launch bound: 1024 threads (4 waves per SIMD, up to 128 VGPRs) where only
-// the cells are in registers (the register variant without adaptive substeps:
-// ~90 VGPRs in 2D, ~120 in 3D; the trail up to 64 steps: ~100 and ~122); 768
-// (3 waves per SIMD, up to 168 VGPRs) for the longer trail, the segmented
-// variant and the adaptive register variant, whose trajectory takes D x 50
-// VGPRs.
-template <bool ADAPTIVE, int BODY>
-constexpr int kBwdThreads = (BODY == kBodyTrail64 || (BODY == kBodyRegister && !ADAPTIVE)) ? 1024 : 768;
+// Launch bound: 1024 threads (4 waves per SIMD, up to 128 VGPRs) for the
+// register variant without adaptive substeps, which keeps only the cells (111
+// to 115 VGPRs in 2D, 126 to 128 in 3D); trail_lanes for the trail; 768 (3 waves
+// per SIMD, up to 168 VGPRs) for the segmented variant and the adaptive register
+// variant, whose trajectory takes D x 50 VGPRs.
+template <int D, bool ADAPTIVE, int BODY>
+constexpr int kBwdThreads = is_trail(BODY) ? trail_lanes(D, BODY == kBodyTrail64 ? 64 : 104)
+                            : (BODY == kBodyRegister && !ADAPTIVE) ? 1024 : 768;
 
 template <int D, bool ADAPTIVE, bool LDS_A, int BINS, int BODY>
-__global__ __launch_bounds__((kBwdThreads<ADAPTIVE, BODY>)) void backward_kernel(
+__global__ __launch_bounds__((kBwdThreads<D, ADAPTIVE, BODY>)) void backward_kernel(
     int nP, int batched, int T, Cells g, int nC, int K, const float* __restrict__ points,
     const float* __restrict__ stage_points, const float* __restrict__ As,
     const float* __restrict__ Gs, Recover rec, const float* __restrict__ grad_out,
@@ -128,7 +129,7 @@ __global__ __launch_bounds__((kBwdThreads<ADAPTIVE, BODY>)) void backward_kernel
 // each value save (16 x 10,000 points, one channel: whole pass 36.3 us here, 40.1
 // with the scatter apart; three channels 48.3 and 52.9).
 template <int D, bool ADAPTIVE, bool LDS_A, int BINS, int BODY, typename GS>
-__global__ __launch_bounds__((kBwdThreads<ADAPTIVE, BODY>)) void image_backward_kernel(
+__global__ __launch_bounds__((kBwdThreads<D, ADAPTIVE, BODY>)) void image_backward_kernel(
     ImageShape s, int T, Cells g, int nC, const float* __restrict__ axes,
     const float* __restrict__ final_points, const float* __restrict__ seed_grad,
     const float* __restrict__ As,
@@ -178,8 +179,7 @@ hipError_t go(const BackwardJob& j, const LaunchCfg& cfg, hipStream_t s) {
   const size_t lds = stage_lds_bytes<D, LDS_A, BINS>(j.geo.nC);
   const Cells g{j.geo.nx, j.geo.ny, j.geo.nz};
   const Recover rec{j.amp, adjoint_table_blocks(j.geo.nC),
-                    (float)std::pow((double)kRecoverGrowth,
-                                    1.0 / (double)(is_trail(BODY) ? std::min(j.T, kSeg) : j.T)),
+                    (float)std::pow((double)kRecoverGrowth, 1.0 / (double)j.T),
                     j.edge};
   const dim3 grid((unsigned)cfg.chunks, (unsigned)j.n_batch), block((unsigned)cfg.block);
   // Doubles serve single transforms of point arrays, and those always (see Bins).

@@ -547,8 +547,8 @@ __device__ __forceinline__ void register_body(P tab, PG gtab, int nP, const Cell
                                               const IO& io, const Sink& flush, float delta) {
   constexpr int PP = Dim<D>::P;
   // A trajectory's last flush has all 64 lanes of every wave adding to
-  // scattered bins at the same moment, a burst the LDS atomic pipe drains at
-  // about one lane per clock.  With full bins (1D/2D, no adaptive substeps:
+  // scattered bins at the same moment, a burst that the LDS atomic pipe drains in
+  // the cycles given at Bins.  With full bins (1D/2D, no adaptive substeps:
   // registers to spare) it is kept pending instead and issued one component
   // every TS / PP steps during the next range's phase 1, alongside its VALU
   // work; the last range's flush follows the loop.
@@ -710,17 +710,18 @@ template <> struct Trail<104> {
   }
 };
 
-// register_body without adaptive substeps for any T <= CAP.  Each whole group's
-// start position is kept too, and phase 2 takes it up again at the group's end,
-// so a recovered position is at most kSeg steps of rounding away from the
-// replayed one (without that, the theta gradient of a [48, 48] field was three
-// times further from its 64-bit value), and a row need only keep the growth
-// bound over kSeg steps, or over T if those are fewer.
+// The backward without adaptive substeps for any T <= CAP.  Each whole group's
+// start position is kept beside the cells, and phase 2 replays the group's
+// positions from it over those cells: the same positions as phase 1's, bit for bit,
+// with no bound on the field.  (Recovering them through the inverse maps, as
+// register_body does over its 50 steps, is 3 to 13 % faster up to 64 steps, but
+// theta's gradient was up to 1.7 times further from its 64-bit value than the
+// segmented body's: 4 rows of 10,000 points, [50], T = 20, 7.1e-6 against 4.8e-6.)
 // Bound by VALU issue and the latency of cell changes, as register_body.  One
-// midpoint pass and table reads only at cell changes, where the segmented body
-// makes two passes and reads an entry at every step: 16 thetas x 60,001 points,
-// [16, 16], T = 20: 118 -> 75 us; 2 x 400,000 points, [48, 48] (LDS cell
-// cache), T = 50: 701 -> 211 us.
+// look-up pass and table reads only at cell changes, where the segmented body
+// looks every step up twice and reads an entry at every step (segmented and trail):
+// 16 x 60,001 points, [16, 16], T = 20, 155 and 105 us; 2 x 400,000, [48, 48] (LDS
+// cell cache), T = 50, 744 and 202; 8 x 40,000, [5, 5, 5], T = 20, 141 and 74.
 template <int D, int CAP, typename P, typename PG, typename IO, typename Sink>
 __device__ __forceinline__ void trail_body(P tab, PG gtab, int nP, int T, const Cells& g,
                                            const IO& io, const Sink& flush, float delta) {
@@ -814,42 +815,71 @@ __device__ __forceinline__ void trail_body(P tab, PG gtab, int nP, int T, const 
 #pragma unroll
     for (int k = 0; k < PP; ++k) m[k] = 0.0f;
     Adj<D> G = fetch_adj<D>(gtab, c);
-    Inv<D> E = fetch_inv<D>(gtab, c);
-    auto back = [&](uint32_t cell) {
-      const int cn = (int)cell;
+    auto back = [&](int cn, const float (&at)[D]) {
       // Divergent branch, skipped where no lane changes cell; the next cell's
       // entry is read before the finished cell's sums are added (LDS operations
       // retire in order).
       if (__builtin_expect(cn != c, 0)) {
         G = fetch_adj<D>(gtab, cn);
-        E = fetch_inv<D>(gtab, cn);
         if (valid) flush(c, m);
 #pragma unroll
         for (int k = 0; k < PP; ++k) m[k] = 0.0f;
       }
       c = cn;
-      step_back<D>(E, p);  // p = position at this step
-      adjoint(G, p, m, lam);
+      adjoint(G, at, m, lam);
       // The lambda update reads G: finish it before a branch that reloads G.
       pin(lam);
     };
-#pragma unroll 1
-    for (int q = groups - 1; q >= 0; --q) {
+    // A group's n steps (uniform) replayed from p, its start, and then backwards.
+    auto sweep = [&](int word, auto n) {
       uint32_t w[kTrailWords];
 #pragma unroll
-      for (int k = 0; k < kTrailWords; ++k) w[k] = trail.get(word0 + kTrailWords * q + k);
+      for (int k = 0; k < kTrailWords; ++k) w[k] = trail.get(word + k);
+      auto cell = [&](int k) { return (int)((k & 1) ? w[k / 2] >> 16 : w[k / 2] & 0xffffu); };
+      float x[kSeg][D];
+      Aff<D> A;
+      int at = -1;
 #pragma unroll
-      for (int k = kTrailWords - 1; k >= 0; --k) {
-        back(w[k] >> 16);
-        back(w[k] & 0xffffu);
+      for (int k = 0; k < kSeg; ++k) {
+        if (k < n) {
+#pragma unroll
+          for (int d = 0; d < D; ++d) x[k][d] = p[d];
+          if (k + 1 < n) {
+            const int cn = cell(k);
+            if (__builtin_expect(cn != at, 0)) A = fetch<D>(tab, cn);
+            at = cn;
+            midpoint(A, p, h, hh);
+          }
+        }
       }
 #pragma unroll
+      for (int k = kSeg - 1; k >= 0; --k)
+        if (k < n) back(cell(k), x[k]);
+    };
+    auto start_of = [&](int q) {
+#pragma unroll
       for (int k = 0; k < D; ++k) p[k] = starts[k][q];
-    }
+    };
+    if constexpr (D <= 2) {
+      // n known when this is compiled for the whole groups: [50] x 16 x 100,000
+      // points, T = 64, 148 -> 130 us.
 #pragma unroll 1
-    for (int t = head - 1; t >= 0; --t) {
-      const uint32_t w = trail.get(t >> 1);
-      back((t & 1) ? w >> 16 : w & 0xffffu);
+      for (int q = groups - 1; q >= 0; --q) {
+        start_of(q);
+        sweep(word0 + kTrailWords * q, std::integral_constant<int, kSeg>{});
+      }
+      if (head) {
+        io.start(pi, p);
+        sweep(0, head);
+      }
+    } else {
+      // One copy of the sweep: two spill (236 VGPRs up to 64 steps, none so).
+#pragma unroll 1
+      for (int q = groups - 1; q >= (head ? -1 : 0); --q) {
+        if (q < 0) io.start(pi, p);
+        else start_of(q);
+        sweep(word0 + kTrailWords * q, q < 0 ? head : kSeg);
+      }
     }
     if constexpr (kSpread) {
       wave_run_sums<PP>(valid, c, m, pend, pend_on);
@@ -1007,13 +1037,11 @@ __device__ __forceinline__ void run_stage(const StageLds<D, LDS_A, BINS>& L, con
                                           const IO& io, float* __restrict__ mom_b,
                                           const Recover& rec, size_t row, float delta) {
   const FloatSink<BINS, Dim<D>::P> sink{L.bins, L.keys, mom_b};
-  if constexpr (BODY != kBodySegmented && !ADAPTIVE) {
+  if constexpr (BODY == kBodyRegister && !ADAPTIVE) {
     // Rows whose inverse maps could amplify the recovered positions' rounding
     // beyond kRecoverGrowth replay each segment from a checkpoint instead.
     if (!recover_ok(rec.amp + row * rec.namp, rec.namp, rec.amp_max)) {
-      constexpr int kSteps = BODY == kBodyRegister ? kRegSteps : BODY == kBodyTrail64 ? 64 : 104;
-      segmented_run<D, false, (kSteps + kSeg - 1) / kSeg>(
-          Ag, Gg, nP, BODY == kBodyRegister ? kRegSteps : T, g, io, sink);
+      segmented_run<D, false, (kRegSteps + kSeg - 1) / kSeg>(Ag, Gg, nP, kRegSteps, g, io, sink);
       return;
     }
   }

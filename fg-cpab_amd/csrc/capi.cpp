@@ -157,7 +157,7 @@ enum class Work { kPoints, kChain, kImage };
 // Backward: full LDS bins when a theta's nC x ppc table fits in LDS, else the
 // hashed LDS cell cache (at most 154 KiB, 2D).  Register variant for T = 50
 // and trail variant for other T (cells, and with adaptive substeps at T = 50
-// positions, in VGPRs; one workgroup per CU of 1024 lanes, or 768 for the
+// positions, in VGPRs; one workgroup per CU of 1024 lanes, or fewer for the
 // variants that need more registers); otherwise the segmented variant, with
 // the affine table in LDS beside the bins when both fit.
 // Returns false (message set) if the device's LDS holds neither.
@@ -205,7 +205,7 @@ bool backward_cfg(const cpab::Geometry& g, int64_t nP, int64_t n_theta, int T, i
   const int64_t lds = used + (c.lds_table ? table : 0);
   int wg_per_cu;
   if (reg) {
-    c.block = adaptive || c.trail == 104 ? 768 : 1024;  // the kernel's launch bound
+    c.block = c.trail ? cpab::trail_lanes(g.ndim, c.trail) : adaptive ? 768 : 1024;  // the kernel's launch bound
     wg_per_cu = 1;
   } else {
     // 32 waves per CU as 512-lane workgroups, as many as LDS allows; the cache

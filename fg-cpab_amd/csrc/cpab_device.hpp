@@ -36,11 +36,10 @@ constexpr int kRegSteps = 50;
 // points leave most lanes idle (1 x 5,001 at [36, 36], T = 3, 48.9 and 39.1, T = 8 53.4
 // and 45.9; 32 x 4,001 at [31, 31], T = 8, 101.6 and 106.4).
 constexpr int kFewSteps = 4;
-// The register and trail backwards recover positions step by step through each cell's
+// The register backward recovers positions step by step through each cell's
 // inverse one-step map M_c, which multiplies the rounding error of a recovered
-// position by up to ||M_c||_2 per step.  They do so only for rows (thetas)
-// whose bound (max_c ||M_c||_2)^n is at most kRecoverGrowth over the n steps
-// between known positions (T; trail: at most kSeg); other rows replay
+// position by up to ||M_c||_2 per step.  It does so only for rows (thetas)
+// whose bound (max_c ||M_c||_2)^T is at most kRecoverGrowth; other rows replay
 // the trajectory from checkpoints, which reproduces the replayed positions
 // exactly.  Measured on a CPU emulation of the recovery (1D/2D/3D rows): the
 // largest position error is about 4e-6 below a bound of 2 (theta ~ N(0, 0.5^2),

@@ -45,6 +45,14 @@ constexpr int kInterpTile0 = 32;
 constexpr int kInterpTileLast = 32;
 constexpr int kInterpThreads = 256;
 
+// Lanes of the trail bodies' workgroups, one to a compute unit: as many as leave
+// the cells, a group's positions and the step in VGPRs (up to 64 and up to 104 steps:
+// 1D 91 and 129 of them, 2D 128 and 168 with 12 to 19 spilled, 3D 157 and 202; 3D in
+// 128 and 168 would spill 122 and 250).
+constexpr int trail_lanes(int ndim, int cap) {
+  return ndim <= 2 ? (cap == 64 ? 1024 : 768) : (cap == 64 ? 768 : 512);
+}
+
 // Launch shape, chosen per problem by the C-ABI layer (capi.cpp).
 struct LaunchCfg {
   int block;        // threads per workgroup

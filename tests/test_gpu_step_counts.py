@@ -49,6 +49,13 @@ def test_backward_rounding_many_tables(cuda):
     _check_rounding([50], 1, 1, 60000, cuda)
 
 
+@pytest.mark.parametrize("nstep", [1, 5, 8])
+@pytest.mark.parametrize("tess", [[50], [16, 16], [48, 48], [5, 5, 5]])
+def test_backward_rounding(cuda, tess, nstep):
+    # the reverse sweep's positions are the replay's own
+    _check_rounding(tess, nstep, 4, 10000, cuda)
+
+
 def _check_rounding(tess, nstep, n_theta, n, cuda):
     # The oracle replays the same float positions and adds in double.  What is left is
     # the roundings of the adjoint, one for each step, and those of a workgroup's table,
