@@ -196,8 +196,8 @@ __device__ __forceinline__ float stack_pop(float (&a)[N]) {
 // one-step maps, staged in LDS beside them), or the hashed LDS cell cache.
 //
 // Double because of the LDS atomic unit, not of the rounding: ds_add_f64 takes
-// 9 to 17 cycles for a whole wave, ds_add_f32 3 cycles per active lane (6 for
-// one or two lanes, 194 for 64), and every trajectory ends in a flush of all
+// 7 to 20 cycles for a whole wave, ds_add_f32 3 cycles per active lane (5 for
+// one lane, 192 for 64), and every trajectory ends in a flush of all
 // lanes at once (C2 backward 163 -> 154 us; 16 thetas x 60,001 points, T = 20:
 // 75 -> 57 us; 8 x 40,000 points, [5, 5, 5]: 86 -> 76 us).  Single transforms of
 // point arrays take it where it fits.  The image backward, and chains, whose
