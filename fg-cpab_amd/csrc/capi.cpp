@@ -182,12 +182,13 @@ bool backward_cfg(const cpab::Geometry& g, int64_t nP, int64_t n_theta, int T, i
   const bool unrolled = packs && T == cpab::kRegSteps &&
                         (g.ndim <= 2 ? c.lds_bins != 0 : !adaptive);
   c.reg_steps = unrolled ? cpab::kRegSteps : 0;
-  // Few steps over a 2D table too large for bins of doubles: the trail saves too
-  // little replay for its larger workgroups (kFewSteps).
+  // Few steps over a large 2D table: the trail saves too little replay for its larger
+  // workgroups (kFewSteps).
   const int64_t budget = dev.lds - 512;   // the kernel's own few words
-  const int most = nP * n_theta <= 128LL * dev.cus ? 2 * cpab::kFewSteps : cpab::kFewSteps;
-  const bool few = T <= most && g.ndim == 2 && c.lds_bins && 2 * table > budget &&
-                   work != Work::kChain;
+  const bool idle = nP * n_theta <= 128LL * dev.cus;   // points leave most lanes idle
+  const bool few = g.ndim == 2 && work != Work::kChain &&
+                   (idle ? T <= 2 * cpab::kFewSteps && table >= 32768
+                         : T <= cpab::kFewSteps && c.lds_bins && 2 * table > budget);
   c.trail = packs && !adaptive && !unrolled && !few ? (T <= 64 ? 64 : 104) : 0;
   const bool reg = unrolled || c.trail;
   // Register and trail variants with full bins: bins of doubles when they fit
@@ -202,7 +203,7 @@ bool backward_cfg(const cpab::Geometry& g, int64_t nP, int64_t n_theta, int T, i
                (work == Work::kImage || c.lds_bins64) && g.ndim <= 2 &&
                (c.lds_bins64 ? 2 : 1) * table + rev <= budget) ? 1 : 0;
   const int64_t used = c.lds_bins ? table : cache;
-  c.lds_table = (!reg && used + table <= dev.lds) ? 1 : 0;
+  c.lds_table = (!reg && !few && used + table <= dev.lds) ? 1 : 0;
   const int64_t lds = used + (c.lds_table ? table : 0);
   int wg_per_cu;
   if (reg) {
@@ -461,7 +462,7 @@ int64_t workspace_size_impl(int ndim, int64_t nP, int64_t n_batch, int K, int nC
   // step count and adaptive substeps are not arguments here) at its most steps,
   // spread or not.
   const struct { int T, adaptive; } bodies[] = {
-      {cpab::kRegSteps, 0}, {cpab::kRegSteps, 1}, {64, 0}, {cpab::kMaxSteps, 0}, {1, 1}};
+      {cpab::kRegSteps, 0}, {cpab::kRegSteps, 1}, {64, 0}, {cpab::kMaxSteps, 0}, {1, 0}, {1, 1}};
   int64_t most = 0;
   for (const auto& body : bodies) {
     cpab::LaunchCfg cfg;

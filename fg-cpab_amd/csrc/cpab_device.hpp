@@ -32,9 +32,11 @@ constexpr int kRegSteps = 50;
 // Step counts up to which the segmented body serves 2D tables with full bins of
 // floats ([30, 30] to [41, 41]; whole pass, trail and segmented: 4 x 60,001 points at
 // [41, 41], T = 2, 131.4 and 125.5 us, T = 4 136.6 and 135.4, T = 8 140.2 and 144.3; 8 x
-// 60,001 at [30, 30], T = 2, 66.1 and 63.5, T = 5 71.6 and 74.1); twice as many where the
-// points leave most lanes idle (1 x 5,001 at [36, 36], T = 3, 48.9 and 39.1, T = 8 53.4
-// and 45.9; 32 x 4,001 at [31, 31], T = 8, 101.6 and 106.4).
+// 60,001 at [30, 30], T = 2, 66.1 and 63.5, T = 5 71.6 and 74.1); twice as many, and from
+// tables of 32 KiB, where the points leave most lanes idle (1 x 5,001 at [36, 36], T = 3,
+// 48.9 and 39.1, T = 8 53.4 and 45.9; 32 x 4,001 at [31, 31], T = 8, 101.6 and 106.4; 2 x
+// 10,000 at [20, 20], T = 3, 40.4 and 33.5, T = 8 43.2 and 38.4; at [48, 48], in the cell
+// cache, 46.7 and 43.2, 52.6 and 53.0).
 constexpr int kFewSteps = 4;
 // The register backward recovers positions step by step through each cell's
 // inverse one-step map M_c, which multiplies the rounding error of a recovered

@@ -37,7 +37,10 @@ def test_backward_step_counts_cache_and_strong(cuda, tess, nstep, n, scale):
 
 @pytest.mark.parametrize("tess,nstep,n,scale", [([30, 30], 1, 3000, 0.5), ([30, 30], 4, 20000, 0.5),
                                                 ([30, 30], 5, 20000, 0.5), ([41, 41], 8, 3000, 0.5),
-                                                ([41, 41], 9, 3000, 0.5), ([36, 36], 3, 3000, 6.0)])
+                                                ([41, 41], 9, 3000, 0.5), ([36, 36], 3, 3000, 6.0),
+                                                ([20, 20], 3, 3000, 0.5), ([20, 20], 8, 16384, 0.5),
+                                                ([20, 20], 8, 16385, 0.5), ([19, 19], 1, 3000, 0.5),
+                                                ([18, 18], 1, 3000, 0.5), ([48, 48], 5, 3000, 6.0)])
 def test_backward_few_steps_large_table(cuda, tess, nstep, n, scale):
     # the segmented body without adaptive substeps, and both sides of its line
     _check(tess, nstep, n, scale, cuda)
